@@ -456,7 +456,8 @@ int32_t taa_batch_submit(taa_ctx_t* ctx, int32_t n, const taa_batch_item_t* item
  * Tile shape per plan comes from the context's autotuner table: a single one-size frame takes its
  * class's shape, several take the shape tuned for the largest class of at most their total
  * pixel count (a launch over many frames behaves like one frame of their total size), or the
- * default shape when it resolves 2% fewer texels over the batch's frames. */
+ * default shape when it resolves 2% fewer texels over the batch's frames. Frames on the FP16 kernel with
+ * RGBA16F storage are tiled by the launch's size alone. */
 typedef struct taa_batch_plan taa_batch_plan_t;
 int32_t taa_batch_plan_create(taa_ctx_t* ctx, int32_t n, const taa_batch_item_t* items,
                               int32_t arith, taa_batch_plan_t** out);
@@ -485,7 +486,9 @@ int32_t taa_autotune(taa_ctx_t* ctx, int32_t width, int32_t height, int32_t colo
                      float* best_us);
 /* Force a tile shape for a frame class; index -1 restores the built-in default (with CAS: 30x30,
  * or for frames of fewer 30x30 tiles than the device holds workgroups at once, 30x14 and below
- * 512 such tiles 14x14). */
+ * 512 such tiles 14x14).
+ * The FP16 kernel with RGBA16F storage resolves 32-column regions instead: entries 0 to 3 select one,
+ * two, four and two rows a thread. */
 int32_t taa_tile_shape_select(int32_t width, int32_t height, int32_t color_format, int32_t arith,
                               taa_bool32 cas, int32_t index);
 /* The shape index the table holds for a frame class. */

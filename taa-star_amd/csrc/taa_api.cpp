@@ -87,11 +87,16 @@ int default_shape(int W, int H, bool cas) {
     return taastar::kDefaultShapeCas;
 }
 
-int selected_shape(int W, int H, int fmt, int arith, bool cas) {
+// the table's entry of a class, -1: none
+int tuned_shape(int W, int H, int fmt, int arith, bool cas) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(ClassKey{W, H, fmt, arith, cas ? 1 : 0});
-    if (it != g_tune.end()) return it->second;
-    return default_shape(W, H, cas);
+    return it != g_tune.end() ? it->second : -1;
+}
+
+int selected_shape(int W, int H, int fmt, int arith, bool cas) {
+    const int t = tuned_shape(W, H, fmt, arith, cas);
+    return t >= 0 ? t : default_shape(W, H, cas);
 }
 
 // The shape for a launch over the tiles of several frames: such a launch behaves like one frame of
@@ -230,9 +235,23 @@ int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, in
         if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
         return TAA_OK;
     }
-    int e = (arith == TAA_ARITH_FP16 && taastar::fast_path_supported(fd, U, param_idx))
-                ? taastar::launch_resolve_fast(fd, U, shape, stream)
-                : taastar::launch_resolve(fd, U, shape, arith, stream);
+    int e;
+    if (arith == TAA_ARITH_FP16 && taastar::fast_path_supported(fd, U, param_idx)) {
+        if (fd.color_fmt == TAA_FMT_RGBA16F) {
+            const int form = taastar::window_form(fd, U, param_idx);
+            const int tuned = tuned_shape(fd.W, fd.H, fd.color_fmt, arith, cas);
+            taastar::tile_window(fd, 2);
+            const long long n16 = (long long)fd.tiles_x * fd.tiles_y;
+            taastar::tile_window(fd, 4);
+            const long long n32 = (long long)fd.tiles_x * fd.tiles_y;
+            taastar::tile_window(fd, tuned >= 0 ? taastar::kWindowRows[tuned] : taastar::window_rows(n16, n32, cas, form));
+            e = taastar::launch_window(fd, U, form, stream);
+        } else {
+            e = taastar::launch_resolve_fast(fd, U, shape, stream);
+        }
+    } else {
+        e = taastar::launch_resolve(fd, U, shape, arith, stream);
+    }
     if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
     return TAA_OK;
 }
@@ -813,6 +832,8 @@ static int check_items(taa_ctx_t* c, int n, const taa_batch_item_t* items) {
 struct BatchLayout {
     int shape = 0;  // tile shape of the main launch
     bool cas = false, s16 = false, fast = false;
+    bool window = false;  // the FP16 kernel on FP16 storage (taa_window.hip)
+    int rows = 0;         // ... its rows a thread
     int form = 0;  // the FP16 kernel's form (taastar::fast_path_form): the largest over the frames
     bool prod_main = false, prod_up = false;  // every frame of that launch has the production feature set
     int n_main = 0, total_main = 0;
@@ -890,6 +911,34 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
         L.form = std::max(L.form, f);
     }
     if (L.fast && n_rgba != 0 && n_rgba != L.n_main) L.fast = false;
+    L.window = L.fast && L.s16;
+    if (L.window) {
+        // one form for the launch: that of all frames, or the widest of theirs (a fixed form with another one
+        // runs as the form that reads its options)
+        const int first = taastar::window_form(ents[0].fd, ents[0].U, 0);
+        int widest = 0;
+        bool alike = true;
+        long long n16 = 0, n32 = 0;
+        for (int i = 0; i < L.n_main; ++i) {
+            taastar::FrameDesc& fd = ents[i].fd;
+            const int f = taastar::window_form(fd, ents[i].U, 0);
+            alike = alike && f == first;
+            widest = std::max(widest, f == taastar::kDefault ? (int)taastar::kExtRgba : f);
+            taastar::tile_window(fd, 2);
+            n16 += (long long)fd.tiles_x * fd.tiles_y;
+            taastar::tile_window(fd, 4);
+            n32 += (long long)fd.tiles_x * fd.tiles_y;
+        }
+        L.form = alike ? first : widest;
+        L.rows = taastar::window_rows(n16, n32, L.cas, L.form);
+        L.total_main = 0;
+        for (int i = 0; i < L.n_main; ++i) {
+            taastar::BatchEntry& e = ents[i];
+            taastar::tile_window(e.fd, L.rows);
+            e.tile_begin = L.total_main;
+            L.total_main += e.fd.tiles_x * e.fd.tiles_y;
+        }
+    }
     L.prod_main = !L.fast && L.n_main > 0;
     for (int i = 0; i < L.n_main && L.prod_main; ++i) L.prod_main = taastar::exact_prod_form(ents[i].fd, ents[i].U);
     L.prod_up = L.n_up > 0;
@@ -911,7 +960,8 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
 // The launches of one batched call on `stream` (descriptors already on the device at d_ents).
 static int launch_layout(const taastar::BatchEntry* d_ents, const BatchLayout& L, int arith, void* stream) {
     if (L.n_main) {
-        int le = L.fast ? taastar::launch_batch_fast(d_ents, L.n_main, L.total_main, L.shape, L.cas, L.s16, L.form, stream)
+        int le = L.window ? taastar::launch_window_batch(d_ents, L.n_main, L.total_main, L.rows, L.cas, L.form, stream)
+                 : L.fast ? taastar::launch_batch_fast(d_ents, L.n_main, L.total_main, L.shape, L.cas, L.form, stream)
                         : taastar::launch_batch(d_ents, L.n_main, L.total_main, L.shape, L.cas, L.s16, arith, L.prod_main,
                                                 stream);
         if (le) return le;
@@ -986,7 +1036,7 @@ void plan_free(taa_batch_plan* p) {
 }
 
 bool same_launches(const BatchLayout& a, const BatchLayout& b) {
-    return a.shape == b.shape && a.fast == b.fast && a.form == b.form && a.prod_main == b.prod_main &&
+    return a.shape == b.shape && a.fast == b.fast && a.window == b.window && a.rows == b.rows && a.form == b.form && a.prod_main == b.prod_main &&
            a.prod_up == b.prod_up && a.n_main == b.n_main &&
            a.total_main == b.total_main &&
            a.n_up == b.n_up && a.total_up == b.total_up;

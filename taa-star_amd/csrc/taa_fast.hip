@@ -1,9 +1,10 @@
-// gfx950 throughput kernel of the temporal resolve (TAA_ARITH_FP16): the taa.comp configuration
-// of variance clipping + Catmull-Rom history + simple or closest-depth velocity, with optional
-// clamp/clip, reject-outside, depth rejection (raw or linear), Lottes luma weighting and fused CAS.
+// gfx950 throughput kernel of the temporal resolve (TAA_ARITH_FP16) on FP32 storage, and the choice
+// of the FP16 arithmetic's kernel form for both storages (FP16 storage: taa_window.hip): the taa.comp
+// configuration of variance clipping + Catmull-Rom history + simple or closest-depth velocity, with
+// optional clamp/clip, reject-outside, depth rejection (raw or linear), Lottes luma weighting and fused
+// CAS.
 //
-// Arithmetic: texels stay fp16 (storage format) and enter the Catmull-Rom sums through mixed
-// fp16 x fp32 FMAs, variance moments, rectification and the blend run in fp32 with contraction
+// Arithmetic: filters, variance moments, rectification and the blend run in fp32 with contraction
 // and the hardware reciprocal / square root. Everything that selects a texel -- the closest-depth
 // tap, historyUv = uv - v, the Catmull-Rom base texel floor(uv*size - 0.5), the depth-test texel,
 // the out-of-screen and depth-rejection decisions -- is computed exactly as in the FP32 path
@@ -23,26 +24,22 @@
 namespace taastar {
 namespace {
 
-// staged velocity texel: RG16F / RG32F (VEL4 false) or RGBA16F / RGBA32F (VEL4 true), with the
-// colour storage's precision
-template <bool S16, bool VEL4> struct VelSlot;
-template <> struct VelSlot<true, false> { typedef uint32_t T; };  // RG16F bits
-template <> struct VelSlot<false, false> { typedef float2 T; };   // RG32F
-template <> struct VelSlot<true, true> { typedef uint2 T; };      // RGBA16F bits
-template <> struct VelSlot<false, true> { typedef float4 T; };    // RGBA32F
+// staged velocity texel: RG32F (VEL4 false) or RGBA32F
+template <bool VEL4> struct VelSlot;
+template <> struct VelSlot<false> { typedef float2 T; };
+template <> struct VelSlot<true> { typedef float4 T; };
 
-template <int TW_, int TH_, bool CAS_, bool S16_, bool VEL4_ = false>
+template <int TW_, int TH_, bool CAS_, bool VEL4_ = false>
 struct FGeo {
     static constexpr int TW = TW_, TH = TH_;
-    static constexpr bool CAS = CAS_, S16 = S16_, VEL4 = VEL4_;
+    static constexpr bool CAS = CAS_, VEL4 = VEL4_;
     static constexpr int NT = 256;
     static constexpr int A = CAS ? 2 : 1;
     static constexpr int SW = TW + 2 * A, SH = TH + 2 * A, SP = SW + 1;
     static constexpr int RA = CAS ? 1 : 0;
     static constexpr int RW = TW + 2 * RA, RH = TH + 2 * RA, RP = RW + 1;
-    typedef typename VelSlot<S16, VEL4>::T VelT;
-    // resolved screen texel kept for the fused CAS: the value the stored image would hold
-    typedef typename std::conditional<S16, uint2, float4>::type ResT;
+    typedef typename VelSlot<VEL4>::T VelT;
+    typedef float4 ResT;  // resolved screen texel kept for the fused CAS
     static constexpr int NIT = (RW * RH + NT - 1) / NT;  // resolve iterations per thread
     // LDS: the staged region (Y, Co, Cg and depth in one 16-byte entry per texel, velocity, the uv
     // of the staged columns and rows) during the resolve; afterwards the same bytes hold the
@@ -59,27 +56,11 @@ struct FGeo {
     };
 };
 
-template <bool S16, bool VEL4>
-__device__ __forceinline__ float2 vel_xy(typename VelSlot<S16, VEL4>::T v) {
-    if constexpr (VEL4) {
-        if constexpr (S16) return make_float2(h2f(v.x & 0xffffu), h2f(v.x >> 16));
-        else return make_float2(v.x, v.y);
-    } else {
-        if constexpr (S16) return make_float2(h2f(v & 0xffffu), h2f(v >> 16));
-        else return v;
-    }
-}
+__device__ __forceinline__ float2 vel_xy(float2 v) { return v; }
+__device__ __forceinline__ float2 vel_xy(float4 v) { return make_float2(v.x, v.y); }
 // the whole texel as the resolve reads it: RG formats as (r, g, 0, 1)
-template <bool S16, bool VEL4>
-__device__ __forceinline__ float4 vel_xyzw(typename VelSlot<S16, VEL4>::T v) {
-    if constexpr (VEL4) {
-        if constexpr (S16) return make_float4(h2f(v.x & 0xffffu), h2f(v.x >> 16), h2f(v.y & 0xffffu), h2f(v.y >> 16));
-        else return v;
-    } else {
-        const float2 q = vel_xy<S16, false>(v);
-        return make_float4(q.x, q.y, 0.0f, 1.0f);
-    }
-}
+__device__ __forceinline__ float4 vel_xyzw(float2 v) { return make_float4(v.x, v.y, 0.0f, 1.0f); }
+__device__ __forceinline__ float4 vel_xyzw(float4 v) { return v; }
 
 // GEN: the general configuration (variance or plain min/max box, Catmull-Rom or bilinear history,
 // chosen per launch from the parameter block); without it the kernel is the variance box with
@@ -92,7 +73,6 @@ __device__ __forceinline__ float4 vel_xyzw(typename VelSlot<S16, VEL4>::T v) {
 // register budget
 template <class G, bool INSP, bool GEN, bool EXT>
 __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile, typename G::Smem& sm) {
-    constexpr bool S16 = G::S16;
     const taa_params_t& P = U.param[fd.param_idx];
     const int W = fd.W, H = fd.H;
     const uint32_t pitch = (uint32_t)fd.pitch;
@@ -130,7 +110,7 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
         for (int i = tid; i < G::SW * G::SH; i += G::NT) {
             const int gx = clampi(gx0 + sx, 0, W - 1), gy = clampi(gy0 + sy, 0, H - 1);
             const uint32_t gi = (uint32_t)gy * pitch + (uint32_t)gx;
-            const float4 c = ld_rgba<S16>(fd.color, gi);
+            const float4 c = ld_rgba<false>(fd.color, gi);
             float Y = c.x, Co = c.y, Cg = c.z;
             if (ycocg) {
                 const float t = 0.25f * (c.x + c.z);
@@ -212,21 +192,21 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
                 vo = 0;
                 closest = -1;
             }
-            const float2 v = vel_xy<S16, G::VEL4>(sv[l + vo]);
+            const float2 v = vel_xy(sv[l + vo]);
             hu = uvx - v.x;  // taa.comp:421
             hv = uvy - v.y;
         } else {
             // movers only (mode 1) reads .w of the centre tap; RG formats read w = 1
-            const float4 vc = vel_xyzw<S16, G::VEL4>(sv[l]);
+            const float4 vc = vel_xyzw(sv[l]);
             used_velocity = !(P.mUseVelocityVectors == 0 || (P.mUseVelocityVectors == 1 && vc.w < 0.5f));
             if (used_velocity) {
                 float4 vs = vc;
                 if (closest_mode) {
-                    vs = vel_xyzw<S16, G::VEL4>(sv[l + vo]);
+                    vs = vel_xyzw(sv[l + vo]);
                 } else {
                     closest = -1;
                     if (P.mVelocitySampleMode == 1) {  // taa.comp:398-412: the last tap's xy, not the longest
-                        const float2 q = vel_xy<S16, G::VEL4>(sv[l + G::SP + 1]);
+                        const float2 q = vel_xy(sv[l + G::SP + 1]);
                         vs.x = q.x;
                         vs.y = q.y;
                     }
@@ -265,9 +245,9 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
         const float fbx = floorf(tX), fby = floorf(tY);
         const int kx = to_int(fbx), ky = to_int(fby);
         const bool ghost = EXT && P.mDynamicAntiGhosting != 0;
-        const Hist hs = !cr_hist ? history_bilinear_fast<S16>(fd.history, W, H, (int)pitch, kx, ky, tX - fbx, tY - fby)
-                        : ghost  ? history_cr_fast<S16, true>(fd.history, W, H, (int)pitch, kx, ky, tX - fbx, tY - fby)
-                                 : history_cr_fast<S16, false>(fd.history, W, H, (int)pitch, kx, ky, tX - fbx, tY - fby);
+        const Hist hs = !cr_hist ? history_bilinear_fast<false>(fd.history, W, H, (int)pitch, kx, ky, tX - fbx, tY - fby)
+                        : ghost  ? history_cr_fast<false, true>(fd.history, W, H, (int)pitch, kx, ky, tX - fbx, tY - fby)
+                                 : history_cr_fast<false, false>(fd.history, W, H, (int)pitch, kx, ky, tX - fbx, tY - fby);
         __builtin_amdgcn_s_setprio(0);
         const f3 hrgb = hs.c;
         f3 h = hrgb;
@@ -287,7 +267,7 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
         if (ghost) {
             constexpr float eps = 1e-5f;
             auto mov = [&](int o) {
-                const float4 q = vel_xyzw<S16, G::VEL4>(sv[l + o]);
+                const float4 q = vel_xyzw(sv[l + o]);
                 return (fabsf(q.x) > eps || fabsf(q.y) > eps) && (fabsf(q.w) >= 0.5f);
             };
             const bool movC = mov(0);
@@ -381,18 +361,10 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
         }
 
         const uint32_t gi = (uint32_t)cy * pitch + (uint32_t)cx;
-        // fp16 bits of the result, converted once for the history, the screen and the CAS stage
-        uint2 hb = make_uint2(0u, 0u);
-        if constexpr (S16) hb = make_uint2(pack_f2h(aa.x, aa.y), f2h(aa.z));
         if (owned) {
-            if constexpr (S16) {
-                // history alpha = the dynamic mask (0 or 1: 0x3c00 in fp16); the screen's alpha is 1
-                gstore<uint2>(fd.history_out, gi * 8u, make_uint2(hb.x, hb.y | (write_mask != 0.0f ? 0x3c000000u : 0u)));
-                if constexpr (!G::CAS) gstore<uint2>(fd.screen, gi * 8u, make_uint2(hb.x, hb.y | 0x3c000000u));
-            } else {
-                st_rgba<S16>(fd.history_out, gi, make_float4(aa.x, aa.y, aa.z, write_mask));
-                if constexpr (!G::CAS) st_rgba<S16>(fd.screen, gi, make_float4(aa.x, aa.y, aa.z, 1.0f));
-            }
+            // history alpha = the dynamic mask; the screen's alpha is 1
+            st_rgba<false>(fd.history_out, gi, make_float4(aa.x, aa.y, aa.z, write_mask));
+            if constexpr (!G::CAS) st_rgba<false>(fd.screen, gi, make_float4(aa.x, aa.y, aa.z, 1.0f));
             if (EXT && fd.debug) {  // taa.comp:912-942 (mode 8: no mask here, category 0)
                 float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
                 switch (P.mDebugMode) {
@@ -404,7 +376,7 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
                         break;
                     }
                     case 3: g = make_float4(alpha, alpha, alpha, 0.f); break;
-                    case 4: g = vel_xyzw<S16, G::VEL4>(sv[l]); break;
+                    case 4: g = vel_xyzw(sv[l]); break;
                     case 5: g = make_float4(pixel_speed, 0.f, 0.f, 0.f); break;
                     case 6: g = make_float4(aa.x, aa.y, aa.z, 1.0f); break;
                     case 7: g = make_float4(aa.x, aa.y, aa.z, write_mask); break;
@@ -440,8 +412,7 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
             }
         }
         if constexpr (G::CAS) {
-            if constexpr (S16) keep[it] = hb;
-            else keep[it] = make_float4(aa.x, aa.y, aa.z, 0.0f);
+            keep[it] = make_float4(aa.x, aa.y, aa.z, 0.0f);
         }
     }
 
@@ -465,17 +436,12 @@ __device__ void fast_tile(const FrameDesc& fd, const taa_uniforms_t& U, int tile
             if (px >= fd.x_end || py >= H) continue;
             const int li = (oy + 1) * G::RP + (ox + 1);
             const uint32_t go = (uint32_t)py * pitch + (uint32_t)px;
-            if constexpr (S16) {
-                gstore<uint2>(fd.screen, go * 8u,
-                    cas_filter_h2(sr[li - G::RP], sr[li - 1], sr[li], sr[li + 1], sr[li + G::RP], peak));
-            } else {
-                auto at = [&](int k) {
-                    const float4 q = sr[k];
-                    return f3{q.x, q.y, q.z};
-                };
-                const f3 o = cas_filter_fma(at(li - G::RP), at(li - 1), at(li), at(li + 1), at(li + G::RP), peak);
-                st_rgba<S16>(fd.screen, go, make_float4(o.x, o.y, o.z, 1.0f));
-            }
+            auto at = [&](int k) {
+                const float4 q = sr[k];
+                return f3{q.x, q.y, q.z};
+            };
+            const f3 o = cas_filter_fma(at(li - G::RP), at(li - 1), at(li), at(li + 1), at(li + G::RP), peak);
+            st_rgba<false>(fd.screen, go, make_float4(o.x, o.y, o.z, 1.0f));
         }
     }
 }
@@ -485,20 +451,19 @@ struct FastArgs {
     taa_uniforms_t U;
 };
 
-// Occupancy hint: five waves per SIMD for the extended forms (the RGBA-velocity form on FP16
-// storage then holds 96 VGPRs and 24 bytes of spills instead of 101 VGPRs at four waves: 4K with
-// the reference's defaults 56.7 -> 57.7 Gpix/s); the production form reaches 92 VGPRs unhinted.
-template <int TW, int TH, bool CAS, bool S16, bool INSP, int FORM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FORM == 2 || (FORM == 3 && S16) ? 5 : 1))) void k_resolve_fast(const FastArgs a) {
-    using G = FGeo<TW, TH, CAS, S16, FORM == 3>;
+// Occupancy hint: five waves per SIMD for the extended form with RG velocity; the production form
+// reaches 92 VGPRs unhinted.
+template <int TW, int TH, bool CAS, bool INSP, int FORM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FORM == 2 ? 5 : 1))) void k_resolve_fast(const FastArgs a) {
+    using G = FGeo<TW, TH, CAS, FORM == 3>;
     __shared__ typename G::Smem sm;
     const int n = a.fd.tiles_x * a.fd.tiles_y;
     fast_tile<G, INSP, FORM != 0, FORM >= 2>(a.fd, a.U, xcd_tile(blockIdx.x, n), sm);
 }
 
-template <int TW, int TH, bool CAS, bool S16, int FORM>
+template <int TW, int TH, bool CAS, int FORM>
 __global__ __launch_bounds__(256) void k_resolve_fast_batch(const BatchEntry* __restrict__ entries, int n_entries, int total_tiles) {
-    using G = FGeo<TW, TH, CAS, S16, FORM == 3>;
+    using G = FGeo<TW, TH, CAS, FORM == 3>;
     __shared__ typename G::Smem sm;
     const int t = batch_tile(total_tiles);
     if (t < 0) return;
@@ -509,7 +474,7 @@ __global__ __launch_bounds__(256) void k_resolve_fast_batch(const BatchEntry* __
 // FORM: 0 the production form (variance box, Catmull-Rom, RG velocity, no branch on either),
 // 1 the general form (min/max box or bilinear history), 2 the extended form with RG velocity,
 // 3 the extended form with RGBA velocity
-template <bool CAS, bool S16, bool INSP, int FORM>
+template <bool CAS, bool INSP, int FORM>
 hipError_t launch_fast_t(const FrameDesc& fd, const taa_uniforms_t& U, int shape, hipStream_t st) {
     FastArgs a;
     a.fd = fd;
@@ -517,23 +482,23 @@ hipError_t launch_fast_t(const FrameDesc& fd, const taa_uniforms_t& U, int shape
     const int n = fd.tiles_x * fd.tiles_y;
     constexpr const TileShapeDef* S = CAS ? kShapesCas : kShapesPlain;
     switch (shape) {
-        case 0: hipLaunchKernelGGL((k_resolve_fast<S[0].tw, S[0].th, CAS, S16, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
-        case 1: hipLaunchKernelGGL((k_resolve_fast<S[1].tw, S[1].th, CAS, S16, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
-        case 2: hipLaunchKernelGGL((k_resolve_fast<S[2].tw, S[2].th, CAS, S16, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
-        default: hipLaunchKernelGGL((k_resolve_fast<S[3].tw, S[3].th, CAS, S16, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
+        case 0: hipLaunchKernelGGL((k_resolve_fast<S[0].tw, S[0].th, CAS, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
+        case 1: hipLaunchKernelGGL((k_resolve_fast<S[1].tw, S[1].th, CAS, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
+        case 2: hipLaunchKernelGGL((k_resolve_fast<S[2].tw, S[2].th, CAS, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
+        default: hipLaunchKernelGGL((k_resolve_fast<S[3].tw, S[3].th, CAS, INSP, FORM>), dim3(n), dim3(256), 0, st, a); break;
     }
     return hipGetLastError();
 }
 
-template <bool CAS, bool S16, int FORM>
+template <bool CAS, int FORM>
 hipError_t launch_fast_batch_t(const BatchEntry* e, int n, int total, int shape, hipStream_t st) {
     const int grid = batch_grid(total);
     constexpr const TileShapeDef* S = CAS ? kShapesCas : kShapesPlain;
     switch (shape) {
-        case 0: hipLaunchKernelGGL((k_resolve_fast_batch<S[0].tw, S[0].th, CAS, S16, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
-        case 1: hipLaunchKernelGGL((k_resolve_fast_batch<S[1].tw, S[1].th, CAS, S16, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
-        case 2: hipLaunchKernelGGL((k_resolve_fast_batch<S[2].tw, S[2].th, CAS, S16, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
-        default: hipLaunchKernelGGL((k_resolve_fast_batch<S[3].tw, S[3].th, CAS, S16, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
+        case 0: hipLaunchKernelGGL((k_resolve_fast_batch<S[0].tw, S[0].th, CAS, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
+        case 1: hipLaunchKernelGGL((k_resolve_fast_batch<S[1].tw, S[1].th, CAS, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
+        case 2: hipLaunchKernelGGL((k_resolve_fast_batch<S[2].tw, S[2].th, CAS, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
+        default: hipLaunchKernelGGL((k_resolve_fast_batch<S[3].tw, S[3].th, CAS, FORM>), dim3(grid), dim3(256), 0, st, e, n, total); break;
     }
     return hipGetLastError();
 }
@@ -574,50 +539,56 @@ int fast_path_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx) 
     return (!P.mVarianceClipping || P.mInterpolationMode != 2) ? 1 : 0;
 }
 
-template <bool CAS, bool S16, bool INSP>
+int window_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx) {
+    const taa_params_t& p = U.param[param_idx];
+    const int f = fast_path_form(fd, U, param_idx);
+    const bool set = p.mUseYCoCg && p.mVelocitySampleMode == 2 && p.mDepthCulling && p.mLumaWeightingLottes && p.mRejectOutside;
+    const bool clear = !p.mUseYCoCg && p.mVelocitySampleMode == 0 && !p.mDepthCulling && !p.mLumaWeightingLottes && !p.mRejectOutside;
+    if (f == 0) return set && p.mColorClampingOrClipping == 2 ? kProd : kVar;
+    if (f == 3 && clear && p.mColorClampingOrClipping == 1 && !p.mVarianceClipping && p.mInterpolationMode == 0 &&
+        p.mUseVelocityVectors == 1 && !p.mDynamicAntiGhosting && !p.mVelBasedAlpha && !p.mReduceBlendNearClamp && !fd.debug)
+        return kDefault;
+    return f + 1;  // kGeneral, kExt, kExtRgba
+}
+
+int window_rows(long long n16, long long n32, bool cas, int form) {
+    if (n16 < 800) return 1;
+    return cas && form != kDefault && n32 >= 1280 ? 4 : 2;
+}
+
+template <bool CAS, bool INSP>
 hipError_t launch_fast_g(const FrameDesc& fd, const taa_uniforms_t& U, int shape, hipStream_t st) {
     switch (fast_path_form(fd, U, fd.param_idx)) {
-        case 0: return launch_fast_t<CAS, S16, INSP, 0>(fd, U, shape, st);
-        case 1: return launch_fast_t<CAS, S16, INSP, 1>(fd, U, shape, st);
-        case 2: return launch_fast_t<CAS, S16, INSP, 2>(fd, U, shape, st);
-        default: return launch_fast_t<CAS, S16, INSP, 3>(fd, U, shape, st);
+        case 0: return launch_fast_t<CAS, INSP, 0>(fd, U, shape, st);
+        case 1: return launch_fast_t<CAS, INSP, 1>(fd, U, shape, st);
+        case 2: return launch_fast_t<CAS, INSP, 2>(fd, U, shape, st);
+        default: return launch_fast_t<CAS, INSP, 3>(fd, U, shape, st);
     }
 }
 
 int launch_resolve_fast(const FrameDesc& fd, const taa_uniforms_t& U, int shape, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const bool s16 = fd.color_fmt == TAA_FMT_RGBA16F, cas = fd.cas_on != 0, insp = fd.inspect != nullptr;
+    const bool insp = fd.inspect != nullptr;
     hipError_t e;
-    if (insp) {
-        if (cas) e = s16 ? launch_fast_g<true, true, true>(fd, U, shape, st) : launch_fast_g<true, false, true>(fd, U, shape, st);
-        else e = s16 ? launch_fast_g<false, true, true>(fd, U, shape, st) : launch_fast_g<false, false, true>(fd, U, shape, st);
-    } else {
-        if (cas) e = s16 ? launch_fast_g<true, true, false>(fd, U, shape, st) : launch_fast_g<true, false, false>(fd, U, shape, st);
-        else e = s16 ? launch_fast_g<false, true, false>(fd, U, shape, st) : launch_fast_g<false, false, false>(fd, U, shape, st);
-    }
+    if (fd.cas_on) e = insp ? launch_fast_g<true, true>(fd, U, shape, st) : launch_fast_g<true, false>(fd, U, shape, st);
+    else e = insp ? launch_fast_g<false, true>(fd, U, shape, st) : launch_fast_g<false, false>(fd, U, shape, st);
     return (int)e;
 }
 
-template <bool CAS, bool S16>
+template <bool CAS>
 hipError_t launch_fast_batch_f(const BatchEntry* e, int n, int total, int shape, int form, hipStream_t st) {
     switch (form) {
-        case 0: return launch_fast_batch_t<CAS, S16, 0>(e, n, total, shape, st);
-        case 1: return launch_fast_batch_t<CAS, S16, 1>(e, n, total, shape, st);
-        case 2: return launch_fast_batch_t<CAS, S16, 2>(e, n, total, shape, st);
-        default: return launch_fast_batch_t<CAS, S16, 3>(e, n, total, shape, st);
+        case 0: return launch_fast_batch_t<CAS, 0>(e, n, total, shape, st);
+        case 1: return launch_fast_batch_t<CAS, 1>(e, n, total, shape, st);
+        case 2: return launch_fast_batch_t<CAS, 2>(e, n, total, shape, st);
+        default: return launch_fast_batch_t<CAS, 3>(e, n, total, shape, st);
     }
 }
 
-int launch_batch_fast(const BatchEntry* d_entries, int n_entries, int total_tiles, int shape, bool cas, bool s16, int form,
-                      void* stream) {
+int launch_batch_fast(const BatchEntry* d_entries, int n_entries, int total_tiles, int shape, bool cas, int form, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e;
-    if (cas) e = s16 ? launch_fast_batch_f<true, true>(d_entries, n_entries, total_tiles, shape, form, st)
-                     : launch_fast_batch_f<true, false>(d_entries, n_entries, total_tiles, shape, form, st);
-    else e = s16 ? launch_fast_batch_f<false, true>(d_entries, n_entries, total_tiles, shape, form, st)
-                 : launch_fast_batch_f<false, false>(d_entries, n_entries, total_tiles, shape, form, st);
-    return (int)e;
+    return (int)(cas ? launch_fast_batch_f<true>(d_entries, n_entries, total_tiles, shape, form, st)
+                     : launch_fast_batch_f<false>(d_entries, n_entries, total_tiles, shape, form, st));
 }
-
 
 }  // namespace taastar

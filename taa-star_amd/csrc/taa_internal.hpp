@@ -31,6 +31,7 @@ struct FrameDesc {
     uint32_t cas_peak_bits;   // const1[0] of CasSetup
     int32_t Wl, Hl, pitch_l;  // input (render) size of colour, depth, velocity, previous depth
     int32_t up;               // upsampling path: input size != output size, or mUpsampling
+    int32_t rows;             // window kernel: rows of a column a thread resolves
 };
 
 // The segmentation mask's extra images (taa_segmentation_images_t), pitch resolved.
@@ -50,6 +51,7 @@ struct BatchEntry {
     taa_uniforms_t U;         // the frame's uniforms, inline so the kernel reads them with scalar loads
     int32_t tile_begin;       // prefix sum of tiles of the entries before this one
     int32_t pad;
+    uint64_t pad2;            // entries are whole 16-byte words
 };
 
 // Tile shapes the kernels are instantiated for (output tile, 256 threads per workgroup).
@@ -126,8 +128,33 @@ bool fast_path_supported(const FrameDesc& fd, const taa_uniforms_t& U, int param
 // launch's frames must all have RGBA velocity or none)
 int fast_path_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx);
 int launch_resolve_fast(const FrameDesc& fd, const taa_uniforms_t& U, int shape, void* stream);
-int launch_batch_fast(const BatchEntry* d_entries, int n_entries, int total_tiles, int shape, bool cas, bool s16,
-                      int form, void* stream);
+int launch_batch_fast(const BatchEntry* d_entries, int n_entries, int total_tiles, int shape, bool cas, int form, void* stream);
+
+// The FP16-storage form of that kernel (taa_window.hip): a workgroup resolves a region of 32 columns x
+// 32 rows (fd.rows 4: 256 threads, four rows of a column each) or 16 rows (2: 256 threads, two rows
+// each; 1: 512 threads, one row each), of which fused CAS keeps the inner part.
+inline void tile_window(FrameDesc& fd, int rows) {
+    const int ring = fd.cas_on ? 2 : 0;
+    fd.rows = rows;
+    fd.tiles_x = tiles_for(fd.x_end - fd.x_begin, 32 - ring);
+    fd.tiles_y = tiles_for(fd.H, (rows == 4 ? 32 : 16) - ring);
+}
+// rows a thread of a class whose tile shape was tuned or selected (kShapesCas / kShapesPlain index)
+constexpr int kWindowRows[kNumShapes] = {1, 2, 4, 2};
+// Rows a thread for a launch of n16 workgroups on 16-row regions, n32 on 32-row ones (us a frame, FP16 storage
+// and arithmetic, three states in turn, rows 1 / 2 / 4). A launch that leaves the device part empty takes the most
+// threads: CAS 640x360 7.2 / 7.9 / 9.8, without CAS 800x450 7.3 / 8.0 / 10.2, but CAS 800x450 (891 workgroups)
+// 9.9 / 9.6 / 11.1. With CAS the 32-row region resolves 14% ring texels instead of 22% and wins once its workgroups
+// fill the device (five on each of 256 CUs): 1280x720 16.9 / 16.7 / 19.6, 1600x900 23.9 / 23.0 / 22.8, 3840x2160
+// 119 / 115 / 106. Without CAS there is no ring (2560x1440 55.1 / 45.6 / 47.8), and the reference's default block
+// (bilinear history, no window) is lighter in registers (2560x1440 45.4 / 43.3 / 45.9): both stay at two rows.
+int window_rows(long long n16, long long n32, bool cas, int form);
+// its forms: kProd and kDefault fix every option (the production feature set; the reference's default
+// block with RGBA velocity), the others read theirs per launch
+enum WindowForm { kProd = 0, kVar = 1, kGeneral = 2, kExt = 3, kExtRgba = 4, kDefault = 5 };
+int window_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx);
+int launch_window(const FrameDesc& fd, const taa_uniforms_t& U, int form, void* stream);
+int launch_window_batch(const BatchEntry* d_entries, int n_entries, int total, int rows, bool cas, int form, void* stream);
 
 // Edge-AA fallback on category-1 texels of a segmentation mask (taa_edge_aa.hip).
 int launch_edge_aa(const void* src, const uint32_t* mask, void* dst, int W, int H, int pitch, int seg_pitch, int fmt,
