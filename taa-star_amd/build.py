@@ -32,6 +32,7 @@ SOURCES = [
     ("taa_kernels.hip", "hip"),
     ("taa_fast.hip", "hip"),
     ("taa_window.hip", "hip"),
+    ("taa_upscale.hip", "hip"),
     ("taa_velocity.hip", "hip"),
     ("taa_edge_aa.hip", "hip"),
     ("taa_noalloc.hip", "hip"),

@@ -231,7 +231,7 @@ int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, in
     fd.tiles_y = taastar::tiles_for(fd.H, s.th);
     if (fd.up || U.mUpsampling) {  // upsampling path: the launcher tiles by its form's own shape
         fd.up = 1;
-        const int e = taastar::launch_resolve_up(fd, U, arith, stream);
+        const int e = taastar::upscale_form(fd, U) ? taastar::launch_upscale(fd, U, arith, stream) : taastar::launch_resolve_up(fd, U, arith, stream);
         if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
         return TAA_OK;
     }
@@ -838,6 +838,7 @@ struct BatchLayout {
     bool prod_main = false, prod_up = false;  // every frame of that launch has the production feature set
     int n_main = 0, total_main = 0;
     int n_up = 0, total_up = 0;
+    int up_rows = 0, up_lds = 0;  // every upsampling frame takes the kernel of taa_upscale.hip: its rows a thread and LDS
 };
 
 static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int arith, void* host, BatchLayout& L) {
@@ -943,6 +944,30 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
     for (int i = 0; i < L.n_main && L.prod_main; ++i) L.prod_main = taastar::exact_prod_form(ents[i].fd, ents[i].U);
     L.prod_up = L.n_up > 0;
     for (int i = L.n_main; i < L.n_main + L.n_up && L.prod_up; ++i) L.prod_up = taastar::prod_params(ents[i].fd, ents[i].U);
+    bool upscale = L.n_up > 0;
+    long long n4 = 0;
+    int lds4 = 0;
+    for (int i = L.n_main; i < L.n_main + L.n_up && upscale; ++i) {
+        taastar::FrameDesc& fd = ents[i].fd;
+        upscale = taastar::upscale_form(fd, ents[i].U);
+        const int tx = fd.tiles_x, ty = fd.tiles_y;
+        taastar::tile_upscale(fd, 4);
+        n4 += (long long)fd.tiles_x * fd.tiles_y;
+        fd.tiles_x = tx, fd.tiles_y = ty;
+        lds4 = std::max(lds4, taastar::upscale_lds(fd, 4));
+    }
+    if (upscale) {
+        L.up_rows = taastar::upscale_rows(n4, lds4);
+        L.total_up = 0;
+        for (int i = L.n_main; i < L.n_main + L.n_up; ++i) {
+            taastar::BatchEntry& e = ents[i];
+            taastar::tile_upscale(e.fd, L.up_rows);
+            L.up_lds = std::max(L.up_lds, taastar::upscale_lds(e.fd, L.up_rows));
+            e.tile_begin = L.total_up;
+            L.total_up += e.fd.tiles_x * e.fd.tiles_y;
+        }
+        return TAA_OK;
+    }
     if (L.prod_up && L.cas) {  // the production form's own CAS tile, as in taa_resolve_frame
         const taastar::TileShapeDef sp = shape_def(taastar::kUpShapeCasProd, true);
         L.total_up = 0;
@@ -966,6 +991,8 @@ static int launch_layout(const taastar::BatchEntry* d_ents, const BatchLayout& L
                                                 stream);
         if (le) return le;
     }
+    if (L.n_up && L.up_rows)
+        return taastar::launch_upscale_batch(d_ents + L.n_main, L.n_up, L.total_up, L.up_rows, L.up_lds, L.cas, L.s16, arith, stream);
     if (L.n_up)
         return taastar::launch_batch_up(d_ents + L.n_main, L.n_up, L.total_up, L.cas, L.s16, arith, L.prod_up, stream);
     return 0;
@@ -1039,7 +1066,7 @@ bool same_launches(const BatchLayout& a, const BatchLayout& b) {
     return a.shape == b.shape && a.fast == b.fast && a.window == b.window && a.rows == b.rows && a.form == b.form && a.prod_main == b.prod_main &&
            a.prod_up == b.prod_up && a.n_main == b.n_main &&
            a.total_main == b.total_main &&
-           a.n_up == b.n_up && a.total_up == b.total_up;
+           a.n_up == b.n_up && a.total_up == b.total_up && a.up_rows == b.up_rows && a.up_lds == b.up_lds;
 }
 
 // Capture descriptor upload + the batched launches of a layout for one buffer.

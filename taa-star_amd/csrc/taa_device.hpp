@@ -274,9 +274,8 @@ __device__ float bilinear_f32(const float* img, int W, int H, int pitch, float u
 
 // getCurrentUpsampledColor (taa.comp:222-257), one axis: the jittered input sample position s
 // (input texels) for output texel tc and corner offset o, and whether it lands in tc after scaling
-// by h / l. l, h: input and output size; tj = jitter * l * -1 (input texels).
-__device__ __forceinline__ float upsample_axis(float l, float h, float tj, int tc, float o, bool& hit) {
-    const float sc = h / l;
+// by sc = h / l. l, h: input and output size; tj = jitter * l * -1 (input texels).
+__device__ __forceinline__ float upsample_axis(float l, float h, float sc, float tj, int tc, float o, bool& hit) {
     const float s = floorf(l * ((float)tc + o) / h) + 0.5f + tj;
     hit = to_int(s * sc) == tc;
     return s;
@@ -290,10 +289,10 @@ constexpr float kUpsampleCorner = 0.999999f;  // the second corner offset of the
 // axis whenever each axis has one. Returns the input texel it fetches (floor, clamped to the edge),
 // or -1 when no candidate lands -- or, on the x axis (`x`), when the pick is negative, since the
 // reference tests only foundTc.x >= 0.
-__device__ __forceinline__ int upsample_pick(float l, float h, float tj, int tc, int n, bool x) {
+__device__ __forceinline__ int upsample_pick(float l, float h, float sc, float tj, int tc, int n, bool x) {
     bool h0, h1;
-    const float s0 = upsample_axis(l, h, tj, tc, 0.0f, h0);
-    const float s1 = upsample_axis(l, h, tj, tc, kUpsampleCorner, h1);
+    const float s0 = upsample_axis(l, h, sc, tj, tc, 0.0f, h0);
+    const float s1 = upsample_axis(l, h, sc, tj, tc, kUpsampleCorner, h1);
     const float s = h1 ? s1 : s0;
     if (!(h0 || h1) || (x && !(s >= 0.0f))) return -1;
     return clampi(to_int(floorf(s)), 0, n - 1);

@@ -31,7 +31,8 @@ struct FrameDesc {
     uint32_t cas_peak_bits;   // const1[0] of CasSetup
     int32_t Wl, Hl, pitch_l;  // input (render) size of colour, depth, velocity, previous depth
     int32_t up;               // upsampling path: input size != output size, or mUpsampling
-    int32_t rows;             // window kernel: rows of a column a thread resolves
+    int32_t rows;             // window and upscale kernels: rows of a column a thread resolves
+    float to_u[2], up_scale[2];  // upscale kernel: 1 / input size, output size / input size (x, y)
 };
 
 // The segmentation mask's extra images (taa_segmentation_images_t), pitch resolved.
@@ -72,7 +73,8 @@ constexpr int kSegShapeCas = 0;
 constexpr int kSegShapePlain = kDefaultShapePlain;
 // tile shapes of the upsampling resolve (its LDS holds the staged input rectangle); its production
 // form (fewer registers) takes 30x14 CAS tiles: 1080p -> 4K in the FP16 arithmetic 0.205 ms against
-// 0.232 ms with 14x14 (30x30 and 62x14: 0.261 and 0.267 ms); the general form stays at 14x14
+// 0.232 ms with 14x14 (30x30 and 62x14: 0.261 and 0.267 ms); the general form stays at 14x14. The production
+// form is left the sizes that upscale_form() refuses
 constexpr int kUpShapeCas = 0;
 constexpr int kUpShapeCasProd = 1;
 constexpr int kUpShapePlain = kDefaultShapePlain;
@@ -86,8 +88,8 @@ int launch_resolve(const FrameDesc& fd, const taa_uniforms_t& U, int shape, int 
 // culling, Lottes, outside rejection; no debug or inspect image): the general kernel's arithmetic
 // with the other branches compiled out
 bool exact_prod_form(const FrameDesc& fd, const taa_uniforms_t& U);
-// the same switches, whatever the sizes: launch_resolve_up runs the upsampling kernel's production
-// form when they hold; with seg, the same with mRayTraceAugment set (the masked resolve's
+// the same switches, whatever the sizes: launch_upscale (or, for the sizes it does not take, launch_resolve_up's
+// production form) runs when they hold; with seg, the same with mRayTraceAugment set (the masked resolve's
 // production form, whose mask keeps its own parameters)
 bool prod_params(const FrameDesc& fd, const taa_uniforms_t& U, bool seg = false);
 // the upsampling (TAAU) path: exact FP32 arithmetic, or with TAA_ARITH_FP16 the FP16 path's where no
@@ -155,6 +157,44 @@ enum WindowForm { kProd = 0, kVar = 1, kGeneral = 2, kExt = 3, kExtRgba = 4, kDe
 int window_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx);
 int launch_window(const FrameDesc& fd, const taa_uniforms_t& U, int form, void* stream);
 int launch_window_batch(const BatchEntry* d_entries, int n_entries, int total, int rows, bool cas, int form, void* stream);
+
+// The upsampling resolve with the production feature set, inputs no larger than the output
+// (taa_upscale.hip). A workgroup resolves 32 columns x 8 fd.rows rows, of which fused CAS keeps the inner part.
+inline void tile_upscale(FrameDesc& fd, int rows) {
+    const int ring = fd.cas_on ? 2 : 0;
+    fd.to_u[0] = 1.0f / (float)fd.Wl, fd.to_u[1] = 1.0f / (float)fd.Hl;
+    fd.up_scale[0] = (float)fd.W / (float)fd.Wl, fd.up_scale[1] = (float)fd.H / (float)fd.Hl;
+    fd.rows = rows;
+    fd.tiles_x = tiles_for(fd.x_end - fd.x_begin, 32 - ring);
+    fd.tiles_y = tiles_for(fd.H, 8 * rows - ring);
+}
+constexpr int kUpWindowCols = 48, kUpWindowRows = 12;  // its history window: columns, rows beyond the region's
+// LDS of a tile over a w x h rectangle of input texels, in front of the rectangle's boxes (24 bytes each): the staged
+// rectangle and its horizontal depth samples, then in the same place the history window and the resolved texels
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline int up_box_offset(int w, int h, int rows, bool s16) {
+    const int tex = s16 ? 8 : 12, staged = 384 * h + (s16 ? 20 : 24) * w * h, window = kUpWindowCols * (8 * rows + kUpWindowRows) * tex;
+    const int resolved = 256 * rows * (s16 ? 8 : 16);
+    const int most = staged > window ? staged : window;
+    return ((most > resolved ? most : resolved) + 15) & ~15;
+}
+// Whether it takes this frame: with 1.4 (FP16 storage) or 1.6 (FP32 storage) output texels an input texel, where sharing
+// an input texel's box among them pays for the larger LDS (us, the general kernel's production form and this one: FP16
+// 3840x2160 at 1.15 times the input's size 197 and 210, at 1.2 196 and 182; FP32 1920x1080 at 1.25 68 and 66, at 1.3 68 and
+// 60, 3840x2160 at 1.25 256 and 263).
+bool upscale_form(const FrameDesc& fd, const taa_uniforms_t& U);
+// LDS bytes of any tile of the frame (without the tables)
+int upscale_lds(const FrameDesc& fd, int rows);
+// Rows of a column a thread resolves, of a launch of n4 workgroups and lds4 bytes of LDS on four-row tiles: four, whose
+// ring is 14% of the texels instead of 22%, where they fill the device and five share a CU, else two (us, 2 and 4 rows, FP16:
+// 1280x720 to 3840x2160 124 and 114, 1920x1080 to 3840x2160 128 and 120, 640x360 to 1280x720 (1032 workgroups) 19.9 and
+// 20.6, 1280x720 to 1920x1080 (40 KB) 37.8 and 38.8; exact on FP32 storage: 640x360 to 1920x1080 46.4 and 44.5,
+// 960x540 to 1920x1080 (34 KB) 49.6 and 52.4).
+int upscale_rows(long long n4, int lds4);
+int launch_upscale(const FrameDesc& fd, const taa_uniforms_t& U, int arith, void* stream);
+int launch_upscale_batch(const BatchEntry* d_entries, int n_entries, int total, int rows, int lds, bool cas, bool s16, int arith, void* stream);
 
 // Edge-AA fallback on category-1 texels of a segmentation mask (taa_edge_aa.hip).
 int launch_edge_aa(const void* src, const uint32_t* mask, void* dst, int W, int H, int pitch, int seg_pitch, int fmt,

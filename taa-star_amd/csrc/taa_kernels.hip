@@ -876,8 +876,8 @@ __device__ __forceinline__ void resolve_tile(const FrameDesc& fd_in, const taa_u
                     }
                     (col ? sm.uax : sm.uay)[q * n + j] = ba;
                 } else {
-                    (col ? sm.ucx : sm.ucy)[j] = col ? upsample_pick(lx, hxs, tjx, c, Wl, true)
-                                                     : upsample_pick(ly, hys, tjy, c, Hl, false);
+                    (col ? sm.ucx : sm.ucy)[j] = col ? upsample_pick(lx, hxs, hxs / lx, tjx, c, Wl, true)
+                                                     : upsample_pick(ly, hys, hys / ly, tjy, c, Hl, false);
                 }
             }
         }
