@@ -33,6 +33,7 @@ SOURCES = [
     ("taa_fast.hip", "hip"),
     ("taa_window.hip", "hip"),
     ("taa_upscale.hip", "hip"),
+    ("taa_exact.hip", "hip"),
     ("taa_velocity.hip", "hip"),
     ("taa_edge_aa.hip", "hip"),
     ("taa_noalloc.hip", "hip"),

@@ -250,7 +250,13 @@ int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, in
             e = taastar::launch_resolve_fast(fd, U, shape, stream);
         }
     } else {
-        e = taastar::launch_resolve(fd, U, shape, arith, stream);
+        taastar::FrameDesc p = fd;
+        taastar::tile_production(p, taastar::kProd256x2);
+        if (taastar::exact_prod_form(fd, U) &&
+            (long long)p.tiles_x * p.tiles_y >= taastar::exact_workgroups(cas, fd.color_fmt == TAA_FMT_RGBA16F))
+            e = taastar::launch_exact(p, U, stream);
+        else
+            e = taastar::launch_resolve(fd, U, shape, arith, stream);
     }
     if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
     return TAA_OK;
@@ -836,9 +842,10 @@ struct BatchLayout {
     int rows = 0;         // ... its rows a thread
     int form = 0;  // the FP16 kernel's form (taastar::fast_path_form): the largest over the frames
     bool prod_main = false, prod_up = false;  // every frame of that launch has the production feature set
+    bool exact = false;  // the one-size frames take the exact kernel of taa_exact.hip
     int n_main = 0, total_main = 0;
     int n_up = 0, total_up = 0;
-    int up_rows = 0, up_lds = 0;  // every upsampling frame takes the kernel of taa_upscale.hip: its rows a thread and LDS
+    int up_variant = 0, up_lds = 0;  // every upsampling frame takes the kernel of taa_upscale.hip: its variant and LDS
 };
 
 static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int arith, void* host, BatchLayout& L) {
@@ -944,25 +951,41 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
     for (int i = 0; i < L.n_main && L.prod_main; ++i) L.prod_main = taastar::exact_prod_form(ents[i].fd, ents[i].U);
     L.prod_up = L.n_up > 0;
     for (int i = L.n_main; i < L.n_main + L.n_up && L.prod_up; ++i) L.prod_up = taastar::prod_params(ents[i].fd, ents[i].U);
+    if (L.prod_main) {
+        long long n16 = 0;
+        for (int i = 0; i < L.n_main; ++i) {
+            taastar::FrameDesc fd = ents[i].fd;
+            taastar::tile_production(fd, taastar::kProd256x2);
+            n16 += (long long)fd.tiles_x * fd.tiles_y;
+        }
+        L.exact = n16 >= taastar::exact_workgroups(L.cas, L.s16);
+        if (L.exact) L.total_main = 0;
+        for (int i = 0; i < L.n_main && L.exact; ++i) {
+            taastar::BatchEntry& e = ents[i];
+            taastar::tile_production(e.fd, taastar::kProd256x2);
+            e.tile_begin = L.total_main;
+            L.total_main += e.fd.tiles_x * e.fd.tiles_y;
+        }
+    }
     bool upscale = L.n_up > 0;
-    long long n4 = 0;
-    int lds4 = 0;
+    long long n16 = 0, n32 = 0;
+    int lds32 = 0;
     for (int i = L.n_main; i < L.n_main + L.n_up && upscale; ++i) {
-        taastar::FrameDesc& fd = ents[i].fd;
+        taastar::FrameDesc fd = ents[i].fd;
         upscale = taastar::upscale_form(fd, ents[i].U);
-        const int tx = fd.tiles_x, ty = fd.tiles_y;
-        taastar::tile_upscale(fd, 4);
-        n4 += (long long)fd.tiles_x * fd.tiles_y;
-        fd.tiles_x = tx, fd.tiles_y = ty;
-        lds4 = std::max(lds4, taastar::upscale_lds(fd, 4));
+        taastar::tile_production(fd, taastar::kProd256x2);
+        n16 += (long long)fd.tiles_x * fd.tiles_y;
+        taastar::tile_production(fd, taastar::kProd256x4);
+        n32 += (long long)fd.tiles_x * fd.tiles_y;
+        lds32 = std::max(lds32, taastar::upscale_lds(fd, taastar::kProd256x4));
     }
     if (upscale) {
-        L.up_rows = taastar::upscale_rows(n4, lds4);
+        L.up_variant = taastar::upscale_variant(n16, n32, lds32);
         L.total_up = 0;
         for (int i = L.n_main; i < L.n_main + L.n_up; ++i) {
             taastar::BatchEntry& e = ents[i];
-            taastar::tile_upscale(e.fd, L.up_rows);
-            L.up_lds = std::max(L.up_lds, taastar::upscale_lds(e.fd, L.up_rows));
+            taastar::tile_production(e.fd, L.up_variant);
+            L.up_lds = std::max(L.up_lds, taastar::upscale_lds(e.fd, L.up_variant));
             e.tile_begin = L.total_up;
             L.total_up += e.fd.tiles_x * e.fd.tiles_y;
         }
@@ -986,13 +1009,14 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
 static int launch_layout(const taastar::BatchEntry* d_ents, const BatchLayout& L, int arith, void* stream) {
     if (L.n_main) {
         int le = L.window ? taastar::launch_window_batch(d_ents, L.n_main, L.total_main, L.rows, L.cas, L.form, stream)
+                 : L.exact ? taastar::launch_exact_batch(d_ents, L.n_main, L.total_main, L.cas, L.s16, stream)
                  : L.fast ? taastar::launch_batch_fast(d_ents, L.n_main, L.total_main, L.shape, L.cas, L.form, stream)
                         : taastar::launch_batch(d_ents, L.n_main, L.total_main, L.shape, L.cas, L.s16, arith, L.prod_main,
                                                 stream);
         if (le) return le;
     }
-    if (L.n_up && L.up_rows)
-        return taastar::launch_upscale_batch(d_ents + L.n_main, L.n_up, L.total_up, L.up_rows, L.up_lds, L.cas, L.s16, arith, stream);
+    if (L.n_up && L.up_variant)
+        return taastar::launch_upscale_batch(d_ents + L.n_main, L.n_up, L.total_up, L.up_variant, L.up_lds, L.cas, L.s16, arith, stream);
     if (L.n_up)
         return taastar::launch_batch_up(d_ents + L.n_main, L.n_up, L.total_up, L.cas, L.s16, arith, L.prod_up, stream);
     return 0;
@@ -1063,10 +1087,10 @@ void plan_free(taa_batch_plan* p) {
 }
 
 bool same_launches(const BatchLayout& a, const BatchLayout& b) {
-    return a.shape == b.shape && a.fast == b.fast && a.window == b.window && a.rows == b.rows && a.form == b.form && a.prod_main == b.prod_main &&
+    return a.shape == b.shape && a.fast == b.fast && a.window == b.window && a.rows == b.rows && a.form == b.form && a.prod_main == b.prod_main && a.exact == b.exact &&
            a.prod_up == b.prod_up && a.n_main == b.n_main &&
            a.total_main == b.total_main &&
-           a.n_up == b.n_up && a.total_up == b.total_up && a.up_rows == b.up_rows && a.up_lds == b.up_lds;
+           a.n_up == b.n_up && a.total_up == b.total_up && a.up_variant == b.up_variant && a.up_lds == b.up_lds;
 }
 
 // Capture descriptor upload + the batched launches of a layout for one buffer.

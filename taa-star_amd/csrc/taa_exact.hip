@@ -1,0 +1,263 @@
+// gfx950 exact FP32 resolve with the production feature set (variance box, clip, YCoCg, Catmull-Rom history,
+// closest-depth RG velocity of the colour's precision, depth culling, Lottes, outside rejection; no debug or
+// inspect image), operation for operation that of the general kernel (taa_kernels.hip).
+//
+// What bounds it: VALU issue (about 70% of the time at 1920x1080) and exposed latency. Against the general kernel's
+// tiles: the 4x4 footprint filtered from an LDS window as in taa_window.hip (a thread gathered sixteen 16-byte texels, 256
+// clocks of the CU's vector-memory path a wave); velocity staged; the closest-depth search by rows, which a thread's two
+// rows of one column share; the linear-depth rejection and the clip without their divisions where these cannot matter
+// (linear_depth_reject; |v| <= e), and one test of special values for six quotients by 9 and one for three square roots; 80 and
+// 85 VGPRs instead of 94 and 107, so five or six workgroups a CU. The sums keep taa.comp's order (centre first), so the rows'
+// sums cannot be shared as in the FP16 kernel.
+// us a frame, before and now: FP32 storage with CAS 1920x1080 58.6 and 49.0, 3840x2160 208 and 203, without CAS 1920x1080
+// 52.7 and 42.0, 3840x2160 200 and 168; FP16 storage with CAS 1920x1080 54.2 and 42.8, 3840x2160 186 and 169.
+// Measured and not kept: four rows a thread (1920x1080 with CAS 51.6, 3840x2160 211: four waves a SIMD), 512 threads of two
+// rows (55.7, 235) or of one (54.6; footprints gathered without the window 65.8).
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "taa_device.hpp"
+#include "taa_fast_math.hpp"
+#include "taa_internal.hpp"
+#include "taa_production.hpp"
+#include "taa_wave.hpp"
+
+namespace taastar {
+namespace {
+
+template <bool CAS, bool S16>
+struct ExactGeo : ProdGeo<256, 2, CAS, S16, false> {
+    typedef ProdGeo<256, 2, CAS, S16, false> Base;
+    typedef typename Base::VelT VelT;
+    static constexpr int RW = Base::RW, RH = Base::RH, NT = Base::NT;
+    // staged inputs: the region and one texel around it, two texels of a row a thread, SR rows a pass
+    static constexpr int SW = RW + 2, SH = RH + 2, NS = SW * SH, SC = SW / 2, SR = NT / SC, SP = (SH + SR - 1) / SR;
+    static constexpr int kStaged = NS * (4 + (int)sizeof(VelT)), kWin = Base::WP * Base::WH * (int)sizeof(typename Base::Win),
+                         kRes = RW * RH * Base::TB, kMost = kStaged > kWin ? kStaged : kWin;
+    struct Smem {
+        alignas(16) unsigned char win[kMost > kRes ? kMost : kRes];  // velocity and depth, then the window, then the resolved texels
+        alignas(16) float2 c01[NS];                                  // Y, Co
+        alignas(8) float c2[NS];                                     // Cg
+        float ux[SW], uy[SH];
+        alignas(16) int4 box[NT / 64];
+    };
+};
+
+template <class G>
+__device__ __forceinline__ void resolve_exact(const FrameDesc& fd, const taa_uniforms_t& U, int tile, typename G::Smem& sm) {
+    typedef typename G::VelT VelT;
+    constexpr bool S16 = G::S16;
+    constexpr int RPT = G::RPT, SW = G::SW;
+    const taa_params_t& P = U.param[fd.param_idx];
+    const int W = fd.W, H = fd.H;
+    const uint32_t pitch = (uint32_t)fd.pitch;
+    const int ty = scalar(tile / fd.tiles_x), tx = tile - ty * fd.tiles_x;
+    const int x0 = fd.x_begin + tx * G::TW - G::RA, y0 = ty * G::TH - G::RA;  // the region's first texel
+    const int tid = (int)threadIdx.x, rx = tid & 31, rg = (tid >> 5) * RPT;
+    const float gamma = scalar_now(P.mVarClipGamma), fW = (float)W, fH = (float)H;
+    const Image color(fd.color, fd.pitch, W, H, G::TB), depths(fd.depth, fd.pitch, W, H, 4), velocity(fd.velocity, fd.pitch, W, H, (int)sizeof(VelT)),
+        history(fd.history, fd.pitch, W, H, G::TB), hdepth(fd.hdepth, fd.pitch, W, H, 4);
+    VelT* const sv = reinterpret_cast<VelT*>(sm.win);
+    float* const sd = reinterpret_cast<float*>(sv + G::NS);
+
+    // ---- 1. stage colour, depth and velocity of the region and one texel around it, clamped to the edge
+    {
+        auto store = [&](int i, f3 a, f3 b, uint2 d, VelT v0, VelT v1) {
+            a = rgb_to_ycocg(a), b = rgb_to_ycocg(b);
+            *reinterpret_cast<float4*>(sm.c01 + i) = make_float4(a.x, a.y, b.x, b.y);
+            *reinterpret_cast<float2*>(sm.c2 + i) = make_float2(a.z, b.z);
+            *reinterpret_cast<uint2*>(sd + i) = d;
+            sv[i] = v0;
+            sv[i + 1] = v1;
+        };
+        auto rgb16 = [](uint32_t a, uint32_t b) { return f3{lo16(a), hi16(a), lo16(b)}; };
+        auto rgb32 = [](u32x4 t) { return f3{__uint_as_float(t.x), __uint_as_float(t.y), __uint_as_float(t.z)}; };
+        auto vel32 = [](uint32_t a, uint32_t b) { return make_float2(__uint_as_float(a), __uint_as_float(b)); };
+        auto tables = [&] {  // uv of the columns and rows (taa.comp:131), while the loads are under way
+            if (tid < G::SW) sm.ux[tid] = ((float)clampi(x0 - 1 + tid, 0, W - 1) + 0.5f) / fW;
+            else if (tid >= 64 && tid < 64 + G::SH) sm.uy[tid - 64] = ((float)clampi(y0 - 1 + tid - 64, 0, H - 1) + 0.5f) / fH;
+        };
+        const int sy = tid / G::SC, sx = 2 * (tid - sy * G::SC);
+        const bool inside = x0 >= 1 && y0 >= 1 && x0 + G::RW + 1 <= W && y0 + G::RH + 1 <= H;
+        constexpr int kPass = G::SC * G::SR * 2;
+        if (inside) {  // the pass in the scalar offset
+            const uint32_t o = (uint32_t)sy * pitch + (uint32_t)sx;
+            u32x4 c[G::SP * (S16 ? 1 : 2)], v32[S16 ? 1 : G::SP];
+            uint2 d[G::SP], v16[G::SP];
+#pragma unroll
+            for (int p = 0; p < G::SP; ++p) {  // (an offset past the image reads nothing: no load in a branch)
+                const bool have = tid < G::SC * G::SR && sy + p * G::SR < G::SH;
+                const uint32_t s = (uint32_t)(y0 - 1 + p * G::SR) * pitch + (uint32_t)(x0 - 1);
+                if constexpr (S16) {
+                    c[p] = color.ld4(have ? o * 8u : ~15u, s * 8u);
+                    v16[p] = velocity.ld2(have ? o * 4u : ~15u, s * 4u);
+                } else {
+                    c[2 * p] = color.ld4(have ? o * 16u : ~15u, s * 16u);
+                    c[2 * p + 1] = color.ld4(have ? o * 16u + 16u : ~15u, s * 16u);
+                    v32[p] = velocity.ld4(have ? o * 8u : ~15u, s * 8u);
+                }
+                d[p] = depths.ld2(have ? o * 4u : ~15u, s * 4u);
+            }
+            tables();
+#pragma unroll
+            for (int p = 0; p < G::SP; ++p) {
+                if (tid >= G::SC * G::SR || sy + p * G::SR >= G::SH) break;
+                const int i = 2 * tid + p * kPass;
+                if constexpr (S16) store(i, rgb16(c[p].x, c[p].y), rgb16(c[p].z, c[p].w), d[p], v16[p].x, v16[p].y);
+                else store(i, rgb32(c[2 * p]), rgb32(c[2 * p + 1]), d[p], vel32(v32[p].x, v32[p].y), vel32(v32[p].z, v32[p].w));
+            }
+        } else {  // a tile over the image's border: texel by texel, clamped
+            tables();
+#pragma unroll 1
+            for (int p = 0; p < G::SP; ++p) {
+                if (tid >= G::SC * G::SR || sy + p * G::SR >= G::SH) break;
+                const uint32_t r = (uint32_t)clampi(y0 - 1 + sy + p * G::SR, 0, H - 1) * pitch;
+                const uint32_t g0 = r + (uint32_t)clampi(x0 - 1 + sx, 0, W - 1), g1 = r + (uint32_t)clampi(x0 + sx, 0, W - 1);
+                const uint2 d = make_uint2(depths.ld1(g0 * 4u, 0u), depths.ld1(g1 * 4u, 0u));
+                if constexpr (S16) {
+                    const uint2 a = color.ld2(g0 * 8u, 0u), b = color.ld2(g1 * 8u, 0u);
+                    store(2 * tid + p * kPass, rgb16(a.x, a.y), rgb16(b.x, b.y), d, velocity.ld1(g0 * 4u, 0u), velocity.ld1(g1 * 4u, 0u));
+                } else {
+                    const uint2 a = velocity.ld2(g0 * 8u, 0u), b = velocity.ld2(g1 * 8u, 0u);
+                    store(2 * tid + p * kPass, rgb32(color.ld4(g0 * 16u, 0u)), rgb32(color.ld4(g1 * 16u, 0u)), d, vel32(a.x, a.y), vel32(b.x, b.y));
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    // ---- 2. closest depth, history position and previous depth of the thread's texels
+    ProdTexel q[RPT];
+    int4 bases = make_int4(0x7fffffff, 0x7fffffff, 0x7fffffff, 0x7fffffff);
+    {
+        const int base = rg * SW + rx;
+        struct Row {
+            float d, cd;  // the first smallest depth of the row's three in scan order (strict <), the centre's
+            int i;        // its position
+        };
+        float sum = 0.0f;
+        auto read_row = [&](int t) {
+            const int i = base + t * SW;
+            const float dl = sd[i], dc = sd[i + 1], dr = sd[i + 2];
+            const bool c1 = dc < dl;
+            const float d1 = c1 ? dc : dl;
+            const bool c2 = dr < d1;
+            sum += (dl + dc) + dr;
+            return Row{c2 ? dr : d1, dc, i + (c2 ? 2 : c1 ? 1 : 0)};
+        };
+        const float uvx = sm.ux[rx + 1];
+        Row ra = read_row(0), rb = read_row(1);
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            const float uvy = sm.uy[rg + k + 1];
+            const Row rc = read_row(k + 2);
+            // findClosestUvAndZ_3x3 (taa.comp:371-389): the rows' minima in scan order, strict <
+            const bool c1 = rb.d < ra.d;
+            const float d1 = c1 ? rb.d : ra.d;
+            int best = rc.d < d1 ? rc.i : c1 ? rb.i : ra.i;
+            if (!(sum == sum)) {  // a NaN among the depths read so far: the scan itself, in which only a NaN first tap stays
+                best = base + k * SW;
+                float d = sd[best];
+#pragma unroll 1
+                for (int j = 1; j < 9; ++j) {
+                    const int i = base + (k + j / 3) * SW + j % 3;
+                    const float e = sd[i];
+                    if (e < d) d = e, best = i;
+                }
+            }
+            const float2 v = vel_xy(sv[best]);
+            q[k].expected = rb.cd;
+            q[k].hu = uvx - v.x;
+            q[k].hv = uvy - v.y;
+            // the previous depth under the history position (taa.comp:818)
+            const int dx = med3<0>(to_int(q[k].hu * fW), W - 1), dy = med3<0>(to_int(q[k].hv * fH), H - 1);
+            q[k].pd = __uint_as_float(hdepth.ld1(((uint32_t)dy * pitch + (uint32_t)dx) * 4u, 0u));
+            history_base<false>(q[k], W, H, bases);
+            ra = rb, rb = rc;
+        }
+    }
+    // ---- 3. box and current colour of texel k (called for k = 0, 1, ... in turn): its 3x3 texels, the upper six from the call before
+    f3 n[9];
+    auto read3 = [&](int t, int j) {
+        const int i = (rg + t) * SW + rx;
+#pragma unroll
+        for (int x = 0; x < 3; ++x) n[j + x] = {sm.c01[i + x].x, sm.c01[i + x].y, sm.c2[i + x]};
+    };
+    auto box = [&](int k, f3& c, f3& e, f3& cur, bool& found) {
+        if (k == 0) read3(0, 0), read3(1, 3);
+        read3(k + 2, 6);
+        // centre, then the others in scan order (taa.comp:199-213, 272-281)
+        f3 m1 = n[4] + n[0] + n[1] + n[2] + n[3] + n[5] + n[6] + n[7] + n[8];
+        f3 m2 = n[4] * n[4] + n[0] * n[0] + n[1] * n[1] + n[2] * n[2] + n[3] * n[3] + n[5] * n[5] + n[6] * n[6] + n[7] * n[7] + n[8] * n[8];
+        div9_moments(m1, m2);
+        const f3 mean = m1, var = m2 - mean * mean;
+        const f3 sigma = sqrt3({fmaxf(0.0f, var.x), fmaxf(0.0f, var.y), fmaxf(0.0f, var.z)});
+        const f3 mn = mean - gamma * sigma, mx = mean + gamma * sigma;
+        c = 0.5f * (mx + mn);  // clipAabb's centre and half size (taa.comp:326-327)
+        e = 0.5f * (mx - mn) + f3{1e-7f, 1e-7f, 1e-7f};
+        cur = n[4];
+        found = true;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) n[j] = n[j + 3];
+    };
+    finish<G>(fd, U, P, history, x0, y0, q, bases, sm.win, sm.box, box);
+}
+
+struct ResolveArgs {
+    FrameDesc fd;
+    taa_uniforms_t U;
+};
+
+constexpr int exact_waves(bool s16) { return s16 ? 6 : 5; }  // occupancy hint (waves per SIMD): what the LDS of the tile allows
+
+template <bool CAS, bool S16>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(exact_waves(S16)))) void k_resolve_exact(const ResolveArgs a) {
+    using G = ExactGeo<CAS, S16>;
+    __shared__ typename G::Smem sm;
+    resolve_exact<G>(a.fd, a.U, xcd_tile((int)blockIdx.x, a.fd.tiles_x * a.fd.tiles_y), sm);
+}
+
+// the frames of a batch, walked like the other batched kernels
+template <bool CAS, bool S16>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(exact_waves(S16)))) void k_resolve_exact_batch(const BatchEntry* __restrict__ entries, int n_entries, int total) {
+    using G = ExactGeo<CAS, S16>;
+    __shared__ typename G::Smem sm;
+    const int t = batch_tile(total);
+    if (t < 0) return;
+    const BatchEntry& e = batch_entry(entries, n_entries, t);
+    resolve_exact<G>(e.fd, e.U, t - e.tile_begin, sm);
+}
+
+}  // namespace
+
+int launch_exact(const FrameDesc& fd, const taa_uniforms_t& U, void* stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    ResolveArgs a;
+    a.fd = fd;
+    a.U = U;
+    const dim3 g(fd.tiles_x * fd.tiles_y);
+    const bool s16 = fd.color_fmt == TAA_FMT_RGBA16F;
+    if (fd.cas_on) {
+        if (s16) hipLaunchKernelGGL((k_resolve_exact<true, true>), g, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((k_resolve_exact<true, false>), g, dim3(256), 0, st, a);
+    } else {
+        if (s16) hipLaunchKernelGGL((k_resolve_exact<false, true>), g, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((k_resolve_exact<false, false>), g, dim3(256), 0, st, a);
+    }
+    return (int)hipGetLastError();
+}
+
+int launch_exact_batch(const BatchEntry* e, int n, int total, bool cas, bool s16, void* stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const dim3 g(batch_grid(total));
+    if (cas) {
+        if (s16) hipLaunchKernelGGL((k_resolve_exact_batch<true, true>), g, dim3(256), 0, st, e, n, total);
+        else hipLaunchKernelGGL((k_resolve_exact_batch<true, false>), g, dim3(256), 0, st, e, n, total);
+    } else {
+        if (s16) hipLaunchKernelGGL((k_resolve_exact_batch<false, true>), g, dim3(256), 0, st, e, n, total);
+        else hipLaunchKernelGGL((k_resolve_exact_batch<false, false>), g, dim3(256), 0, st, e, n, total);
+    }
+    return (int)hipGetLastError();
+}
+
+}  // namespace taastar

@@ -158,25 +158,37 @@ int window_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx);
 int launch_window(const FrameDesc& fd, const taa_uniforms_t& U, int form, void* stream);
 int launch_window_batch(const BatchEntry* d_entries, int n_entries, int total, int rows, bool cas, int form, void* stream);
 
-// The upsampling resolve with the production feature set, inputs no larger than the output
-// (taa_upscale.hip). A workgroup resolves 32 columns x 8 fd.rows rows, of which fused CAS keeps the inner part.
-inline void tile_upscale(FrameDesc& fd, int rows) {
+// The kernels with the production feature set (taa_exact.hip, taa_upscale.hip): a workgroup resolves a region of 32
+// columns x 16 rows (512 threads of one row of a column, or 256 of two) or 32 rows (512 of two, 256 of four), of which
+// fused CAS keeps the inner part. fd.rows holds the variant.
+enum ProdVariant { kProd512x1 = 1, kProd256x2 = 2, kProd512x2 = 3, kProd256x4 = 4 };
+inline int production_rows(int variant) { return variant >= kProd512x2 ? 32 : 16; }
+inline void tile_production(FrameDesc& fd, int variant) {
     const int ring = fd.cas_on ? 2 : 0;
+    fd.rows = variant;
     fd.to_u[0] = 1.0f / (float)fd.Wl, fd.to_u[1] = 1.0f / (float)fd.Hl;
     fd.up_scale[0] = (float)fd.W / (float)fd.Wl, fd.up_scale[1] = (float)fd.H / (float)fd.Hl;
-    fd.rows = rows;
     fd.tiles_x = tiles_for(fd.x_end - fd.x_begin, 32 - ring);
-    fd.tiles_y = tiles_for(fd.H, 8 * rows - ring);
+    fd.tiles_y = tiles_for(fd.H, production_rows(variant) - ring);
 }
-constexpr int kUpWindowCols = 48, kUpWindowRows = 12;  // its history window: columns, rows beyond the region's
+constexpr int kProdWindowCols = 48, kProdWindowRows = 12;  // the history window: columns, rows beyond the region's
+// The exact kernel at one size (kProd256x2 regions), for launches of at least exact_workgroups() of them (us, general kernel's
+// production form and this one: with CAS 640x360 (572) FP32 storage 8.9 and 10.8, FP16 9.2 and 10.1, 960x540 (1248) 17.9 and
+// 15.6, 18.9 and 15.1; without CAS FP32 960x540 (1020) 12.7 and 13.8, 1280x720 (1800) 19.6 and 19.6, FP16 640x360 (460) 7.8
+// and 8.1, 960x540 13.2 and 12.2): below, most of a workgroup's time is the chain of its loads and barriers, which the
+// general kernel's small tiles keep shorter.
+int launch_exact(const FrameDesc& fd, const taa_uniforms_t& U, void* stream);
+int launch_exact_batch(const BatchEntry* d_entries, int n_entries, int total, bool cas, bool s16, void* stream);
+inline long long exact_workgroups(bool cas, bool s16) { return cas || s16 ? 900 : 1500; }
+// The upsampling resolve, inputs no larger than the output.
 // LDS of a tile over a w x h rectangle of input texels, in front of the rectangle's boxes (24 bytes each): the staged
 // rectangle and its horizontal depth samples, then in the same place the history window and the resolved texels
 #if defined(__HIPCC__)
 __host__ __device__
 #endif
 inline int up_box_offset(int w, int h, int rows, bool s16) {
-    const int tex = s16 ? 8 : 12, staged = 384 * h + (s16 ? 20 : 24) * w * h, window = kUpWindowCols * (8 * rows + kUpWindowRows) * tex;
-    const int resolved = 256 * rows * (s16 ? 8 : 16);
+    const int tex = s16 ? 8 : 12, staged = 384 * h + (s16 ? 20 : 24) * w * h, window = kProdWindowCols * (rows + kProdWindowRows) * tex;
+    const int resolved = 32 * rows * (s16 ? 8 : 16);
     const int most = staged > window ? staged : window;
     return ((most > resolved ? most : resolved) + 15) & ~15;
 }
@@ -186,15 +198,16 @@ inline int up_box_offset(int w, int h, int rows, bool s16) {
 // 60, 3840x2160 at 1.25 256 and 263).
 bool upscale_form(const FrameDesc& fd, const taa_uniforms_t& U);
 // LDS bytes of any tile of the frame (without the tables)
-int upscale_lds(const FrameDesc& fd, int rows);
-// Rows of a column a thread resolves, of a launch of n4 workgroups and lds4 bytes of LDS on four-row tiles: four, whose
-// ring is 14% of the texels instead of 22%, where they fill the device and five share a CU, else two (us, 2 and 4 rows, FP16:
-// 1280x720 to 3840x2160 124 and 114, 1920x1080 to 3840x2160 128 and 120, 640x360 to 1280x720 (1032 workgroups) 19.9 and
-// 20.6, 1280x720 to 1920x1080 (40 KB) 37.8 and 38.8; exact on FP32 storage: 640x360 to 1920x1080 46.4 and 44.5,
-// 960x540 to 1920x1080 (34 KB) 49.6 and 52.4).
-int upscale_rows(long long n4, int lds4);
+int upscale_lds(const FrameDesc& fd, int variant);
+// The variant of a launch of n16 and n32 workgroups on 16- and 32-row regions, the latter's tiles of lds bytes of LDS
+// (us, FP16 storage and arithmetic unless said otherwise): small launches take the most threads (640x360 from 320x180 9.0,
+// 256 threads of two rows 9.5). 32 rows have 14% ring texels instead of 22%, once they fill the device: 512 threads of two rows where three
+// workgroups' LDS fits a CU (1280x720 to 1920x1080 33.4, 16 rows 37.0; exact on FP32 storage 51.7 and 54.5; at a scale of
+// 1.2, where it does not, 45.6 and 43.0), 256 of four where five do, which is at scales of about 2 and more (640x360 to
+// 1920x1080 29.8, 512 threads 31.2; 1280x720 to 3840x2160 110 and 122).
+int upscale_variant(long long n16, long long n32, int lds);
 int launch_upscale(const FrameDesc& fd, const taa_uniforms_t& U, int arith, void* stream);
-int launch_upscale_batch(const BatchEntry* d_entries, int n_entries, int total, int rows, int lds, bool cas, bool s16, int arith, void* stream);
+int launch_upscale_batch(const BatchEntry* d_entries, int n_entries, int total, int variant, int lds, bool cas, bool s16, int arith, void* stream);
 
 // Edge-AA fallback on category-1 texels of a segmentation mask (taa_edge_aa.hip).
 int launch_edge_aa(const void* src, const uint32_t* mask, void* dst, int W, int H, int pitch, int seg_pitch, int fmt,
