@@ -236,15 +236,18 @@ int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, in
         return TAA_OK;
     }
     int e;
-    if (arith == TAA_ARITH_FP16 && taastar::fast_path_supported(fd, U, param_idx)) {
+    const bool fast = arith == TAA_ARITH_FP16 && taastar::fast_path_supported(fd, U, param_idx);
+    const bool exact_default = arith == TAA_ARITH_FP32 && taastar::default_exact_form(fd, U, param_idx);
+    if (fast || exact_default) {
         if (fd.color_fmt == TAA_FMT_RGBA16F) {
-            const int form = taastar::window_form(fd, U, param_idx);
+            const int form = exact_default ? taastar::kDefaultExact : taastar::window_form(fd, U, param_idx);
             const int tuned = tuned_shape(fd.W, fd.H, fd.color_fmt, arith, cas);
             taastar::tile_window(fd, 2);
             const long long n16 = (long long)fd.tiles_x * fd.tiles_y;
             taastar::tile_window(fd, 4);
             const long long n32 = (long long)fd.tiles_x * fd.tiles_y;
             taastar::tile_window(fd, tuned >= 0 ? taastar::kWindowRows[tuned] : taastar::window_rows(n16, n32, cas, form));
+            if (exact_default && fd.rows == 4) taastar::tile_window(fd, 2);
             e = taastar::launch_window(fd, U, form, stream);
         } else {
             e = taastar::launch_resolve_fast(fd, U, shape, stream);
@@ -919,17 +922,19 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
         L.form = std::max(L.form, f);
     }
     if (L.fast && n_rgba != 0 && n_rgba != L.n_main) L.fast = false;
-    L.window = L.fast && L.s16;
+    bool exact_default = arith == TAA_ARITH_FP32 && L.n_main > 0;
+    for (int i = 0; i < L.n_main && exact_default; ++i) exact_default = taastar::default_exact_form(ents[i].fd, ents[i].U, 0);
+    L.window = (L.fast && L.s16) || exact_default;
     if (L.window) {
         // one form for the launch: that of all frames, or the widest of theirs (a fixed form with another one
         // runs as the form that reads its options)
-        const int first = taastar::window_form(ents[0].fd, ents[0].U, 0);
+        const int first = exact_default ? (int)taastar::kDefaultExact : taastar::window_form(ents[0].fd, ents[0].U, 0);
         int widest = 0;
         bool alike = true;
         long long n16 = 0, n32 = 0;
         for (int i = 0; i < L.n_main; ++i) {
             taastar::FrameDesc& fd = ents[i].fd;
-            const int f = taastar::window_form(fd, ents[i].U, 0);
+            const int f = exact_default ? (int)taastar::kDefaultExact : taastar::window_form(fd, ents[i].U, 0);
             alike = alike && f == first;
             widest = std::max(widest, f == taastar::kDefault ? (int)taastar::kExtRgba : f);
             taastar::tile_window(fd, 2);

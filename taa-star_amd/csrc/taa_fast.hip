@@ -551,9 +551,13 @@ int window_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx) {
     return f + 1;  // kGeneral, kExt, kExtRgba
 }
 
+bool default_exact_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx) {
+    return fd.color_fmt == TAA_FMT_RGBA16F && !fd.inspect && fast_path_supported(fd, U, param_idx) && window_form(fd, U, param_idx) == kDefault;
+}
+
 int window_rows(long long n16, long long n32, bool cas, int form) {
     if (n16 < 800) return 1;
-    return cas && form != kDefault && n32 >= 1280 ? 4 : 2;
+    return cas && form < kDefault && n32 >= 1280 ? 4 : 2;
 }
 
 template <bool CAS, bool INSP>

@@ -153,8 +153,13 @@ constexpr int kWindowRows[kNumShapes] = {1, 2, 4, 2};
 int window_rows(long long n16, long long n32, bool cas, int form);
 // its forms: kProd and kDefault fix every option (the production feature set; the reference's default
 // block with RGBA velocity), the others read theirs per launch
-enum WindowForm { kProd = 0, kVar = 1, kGeneral = 2, kExt = 3, kExtRgba = 4, kDefault = 5 };
+enum WindowForm { kProd = 0, kVar = 1, kGeneral = 2, kExt = 3, kExtRgba = 4, kDefault = 5, kDefaultExact = 6 };
 int window_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx);
+// whether kDefaultExact takes a frame of the exact arithmetic: the reference's default block on RGBA16F storage with RGBA16F
+// velocity, no debug or inspect image. The general kernel read its switches per launch (118 VGPRs) and resolved a row of
+// its tile at a time; 1920x1080 with CAS takes 25.3 us now against 55.3, 640x360 6.6 against 7.9 (the cost of a launch),
+// 3840x2160 92 against 194
+bool default_exact_form(const FrameDesc& fd, const taa_uniforms_t& U, int param_idx);
 int launch_window(const FrameDesc& fd, const taa_uniforms_t& U, int form, void* stream);
 int launch_window_batch(const BatchEntry* d_entries, int n_entries, int total, int rows, bool cas, int form, void* stream);
 

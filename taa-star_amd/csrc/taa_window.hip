@@ -1,4 +1,5 @@
-// gfx950 throughput kernel of the temporal resolve on FP16 storage (TAA_ARITH_FP16, RGBA16F).
+// gfx950 throughput kernel of the temporal resolve on FP16 storage (TAA_ARITH_FP16, RGBA16F), and the
+// reference's default block in the exact arithmetic on that storage.
 //
 // Arithmetic: texels stay fp16 and enter the history filter through mixed fp16 x fp32 FMAs; moments,
 // rectification and the blend run in fp32 with contraction and the hardware reciprocal / square root.
@@ -19,7 +20,8 @@
 // LDS that earlier phases are done with, so five workgroups of 32 x 32 texels share a CU.
 // 3840x2160 with CAS: 106.5 us a frame (365 MB of images, 411 MB of HBM traffic) against 125.6 before (378 MB), five
 // waves per SIMD either way; twelve sessions in one batch 361 against 425 us; the reference's default block at
-// 2560x1440 43.3 against 70.5 us (its switches fixed, bilinear footprints gathered directly).
+// 2560x1440 43.3 against 70.5 us (its switches fixed, bilinear footprints gathered directly), and that block in the exact
+// arithmetic, which differs in the bilinear weights, the blend and the CAS, 25.3 against 55.3 us at 1920x1080.
 // Measured and not kept: strips of rows marched by one wave, neighbours by lane shifts and no LDS (4K 141 us: rows
 // shared by two strips come from beyond the L2 twice, four waves per SIMD leave the loads exposed); 512 threads of
 // two rows (4K 115); tiles walked in column order over 2, 3, 4 or 9 tile rows (no gain).
@@ -38,12 +40,14 @@ namespace {
 
 // FORM (WindowForm): kProd and kDefault are the production feature set and the reference's default
 // block with every switch fixed, kVar the variance box with Catmull-Rom history, kGeneral either box
-// and history, kExt and kExtRgba the per-texel options on RG and RGBA velocity.
+// and history, kExt and kExtRgba the per-texel options on RG and RGBA velocity, kDefaultExact the default block in
+// the exact FP32 arithmetic.
 template <int NT_, int RPT_, bool CAS_, bool INSP_, int FORM_>
 struct WinGeo {
     static constexpr bool CAS = CAS_, INSP = INSP_;
     static constexpr int FORM = FORM_;
-    static constexpr bool PROD = FORM == kProd, DEF = FORM == kDefault;
+    static constexpr bool EX = FORM == kDefaultExact;  // exact FP32 arithmetic (taa.comp's operations, no inspect image)
+    static constexpr bool PROD = FORM == kProd, DEF = FORM == kDefault || EX;
     static constexpr bool EXT = FORM >= kExt, V4 = FORM >= kExtRgba;
     static constexpr int VAR = FORM <= kVar ? 1 : DEF ? 0 : kAny;     // variance box, else minimum / maximum
     static constexpr int CR = FORM <= kVar ? 1 : DEF ? 0 : kAny;      // Catmull-Rom history, else bilinear
@@ -534,6 +538,11 @@ __device__ __forceinline__ void resolve_window(const FrameDesc& fd, const taa_un
             const float fx = q[k].fx, fy = q[k].fy, ux = 1.0f - fx, uy = 1.0f - fy;
             auto mix = [](float a, float b, float u, float t) { return __builtin_fmaf(b, t, a * u); };
             auto quad = [&](float a, float b, float c, float d) { return mix(mix(a, b, ux, fx), mix(c, d, ux, fx), uy, fy); };
+            if constexpr (G::EX) {  // bilinear4_quad
+                auto exact = [&](float a, float b, float c, float d) { return (a * ux + b * fx) * uy + (c * ux + d * fx) * fy; };
+                hrgb = {exact(lo16(e[0].x), lo16(e[1].x), lo16(e[2].x), lo16(e[3].x)), exact(hi16(e[0].x), hi16(e[1].x), hi16(e[2].x), hi16(e[3].x)),
+                        exact(lo16(e[0].y), lo16(e[1].y), lo16(e[2].y), lo16(e[3].y))};
+            } else
             hrgb = {quad(lo16(e[0].x), lo16(e[1].x), lo16(e[2].x), lo16(e[3].x)), quad(hi16(e[0].x), hi16(e[1].x), hi16(e[2].x), hi16(e[3].x)),
                     quad(lo16(e[0].y), lo16(e[1].y), lo16(e[2].y), lo16(e[3].y))};
             if (ghost) ha = quad(hi16(e[0].y), hi16(e[1].y), hi16(e[2].y), hi16(e[3].y));
@@ -617,6 +626,7 @@ __device__ __forceinline__ void resolve_window(const FrameDesc& fd, const taa_un
         if (reset) alpha = 1.0f;
         f3 aa = {__builtin_fmaf(alpha, c.x - h.x, h.x), __builtin_fmaf(alpha, c.y - h.y, h.y), __builtin_fmaf(alpha, c.z - h.z, h.z)};
         if (reset) aa = c;  // exactly the current colour, whatever the history holds
+        if constexpr (G::EX) aa = {gmix(h.x, c.x, alpha), gmix(h.y, c.y, alpha), gmix(h.z, c.z, alpha)};
         if (ycocg) {
             const float t = aa.x - aa.z;
             aa = {t + aa.y, aa.x + aa.z, t - aa.y};
@@ -702,7 +712,13 @@ __device__ __forceinline__ void resolve_window(const FrameDesc& fd, const taa_un
                 if (y == 0) u = c;
                 if (y == H - 1) d = c;
             }
-            screen.st2(cas_filter_h2(u, l, c, r, d, peak), out_off, (uint32_t)k * pitch * 8u);
+            if constexpr (G::EX) {
+                auto rgb = [](uint2 t) { return f3{lo16(t.x), hi16(t.x), lo16(t.y)}; };
+                const f3 o = cas_filter(rgb(u), rgb(l), rgb(c), rgb(r), rgb(d), peak);
+                screen.st2(make_uint2(pack_sat(o.x, o.y), pack_sat(o.z, 1.0f)), out_off, (uint32_t)k * pitch * 8u);
+            } else {
+                screen.st2(cas_filter_h2(u, l, c, r, d, peak), out_off, (uint32_t)k * pitch * 8u);
+            }
         }
     }
 }
@@ -744,6 +760,9 @@ void launch_window_f(const FastArgs& a, int form, hipStream_t st) {
         case kGeneral: hipLaunchKernelGGL((k_resolve_window<NT, RPT, CAS, INSP, kGeneral>), n, dim3(NT), 0, st, a); break;
         case kExt: hipLaunchKernelGGL((k_resolve_window<NT, RPT, CAS, INSP, kExt>), n, dim3(NT), 0, st, a); break;
         case kExtRgba: hipLaunchKernelGGL((k_resolve_window<NT, RPT, CAS, INSP, kExtRgba>), n, dim3(NT), 0, st, a); break;
+        case kDefaultExact:
+            if constexpr (!INSP && RPT < 4) hipLaunchKernelGGL((k_resolve_window<NT, RPT, CAS, INSP, kDefaultExact>), n, dim3(NT), 0, st, a);
+            break;
         default: hipLaunchKernelGGL((k_resolve_window<NT, RPT, CAS, INSP, kDefault>), n, dim3(NT), 0, st, a); break;
     }
 }
@@ -757,6 +776,9 @@ void launch_window_batch_f(const BatchEntry* e, int n, int total, int form, hipS
         case kGeneral: hipLaunchKernelGGL((k_resolve_window_batch<NT, RPT, CAS, kGeneral>), grid, dim3(NT), 0, st, e, n, total); break;
         case kExt: hipLaunchKernelGGL((k_resolve_window_batch<NT, RPT, CAS, kExt>), grid, dim3(NT), 0, st, e, n, total); break;
         case kExtRgba: hipLaunchKernelGGL((k_resolve_window_batch<NT, RPT, CAS, kExtRgba>), grid, dim3(NT), 0, st, e, n, total); break;
+        case kDefaultExact:
+            if constexpr (RPT < 4) hipLaunchKernelGGL((k_resolve_window_batch<NT, RPT, CAS, kDefaultExact>), grid, dim3(NT), 0, st, e, n, total);
+            break;
         default: hipLaunchKernelGGL((k_resolve_window_batch<NT, RPT, CAS, kDefault>), grid, dim3(NT), 0, st, e, n, total); break;
     }
 }

@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 from gpu_helpers import assert_same_bits  # noqa: E402
 from test_gpu_upscale import inputs, test_batches_equal_sessions_alone as batches  # noqa: E402
-from taastar import ARITH_FP32, FMT_RGBA16F, FMT_RGBA32F, VEL_RG16F, VEL_RG32F, FrameImages, check, lib  # noqa: E402
+from taastar import (ARITH_FP32, FMT_RGBA16F, FMT_RGBA32F, VEL_RG16F, VEL_RG32F, VEL_RGBA16F, FrameImages, check,  # noqa: E402
+                     default_params, lib)
 from taastar.workloads import cas_for, uniforms_for, workload  # noqa: E402
 
 
@@ -18,6 +19,27 @@ from taastar.workloads import cas_for, uniforms_for, workload  # noqa: E402
 def _need_gpu():
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
+
+
+def both_forms(w, U, W, H, pitch, images, fmt, K):
+    """Screen and history of the frame without and with a debug image."""
+    color, depth, vel, hist, prev = images
+    out = []
+    for general in (False, True):
+        screen, new = torch.zeros_like(hist), torch.zeros_like(hist)
+        debug = torch.zeros(H, pitch, 4, dtype=torch.float16, device="cuda")
+        img = FrameImages()
+        img.color, img.depth, img.velocity = color.data_ptr(), depth.data_ptr(), vel.data_ptr()
+        img.history, img.history_depth = hist.data_ptr(), prev.data_ptr()
+        img.result_history, img.result_screen = new.data_ptr(), screen.data_ptr()
+        img.debug = debug.data_ptr() if general else None
+        img.width, img.height, img.pitch = W, H, pitch
+        img.color_format, img.velocity_format = fmt, w["vel"]
+        check(lib().taa_resolve_frame(C.byref(U), C.byref(img), C.byref(K) if K else None, ARITH_FP32, None))
+        torch.cuda.synchronize()
+        out.append((screen, new))
+    assert_same_bits(out[0][0], out[1][0], "screen")
+    assert_same_bits(out[0][1], out[1][1], "history")
 
 
 # regions are 30 x 14 (CAS) or 32 x 16 texels, 900 to 1500 of them select the kernel; the second size is a texel beyond
@@ -28,28 +50,25 @@ def _need_gpu():
 def test_equals_the_general_form(W, H, motion, odd, fmt):
     for k, (cas, pad, reset, split) in enumerate([(True, 0, 0, 0), (False, 3, 0, 0), (True, 5, 0, W // 3), (True, 0, 1, 0)]):
         print(f"case {W}x{H} fmt {fmt} cas {cas} pad {pad} reset {reset} split {split}", flush=True)
-        pitch = W + pad
-        color, depth, vel, hist, prev = inputs(W, H, W, H, pitch, pitch, fmt, motion, odd, 71 + k)
         w = workload("c2", fmt=fmt, vel=VEL_RG16F if fmt == FMT_RGBA16F else VEL_RG32F)
         U = uniforms_for(w, 1, (0.3 / W, -0.4 / H))
         U.mResetHistory, U.splitScreen, U.splitX = reset, int(split > 0), split
-        K = cas_for(w, W, H) if cas else None
-        out = []
-        for general in (False, True):
-            screen, new = torch.zeros_like(hist), torch.zeros_like(hist)
-            debug = torch.zeros(H, pitch, 4, dtype=torch.float16, device="cuda")
-            img = FrameImages()
-            img.color, img.depth, img.velocity = color.data_ptr(), depth.data_ptr(), vel.data_ptr()
-            img.history, img.history_depth = hist.data_ptr(), prev.data_ptr()
-            img.result_history, img.result_screen = new.data_ptr(), screen.data_ptr()
-            img.debug = debug.data_ptr() if general else None
-            img.width, img.height, img.pitch = W, H, pitch
-            img.color_format, img.velocity_format = fmt, w["vel"]
-            check(lib().taa_resolve_frame(C.byref(U), C.byref(img), C.byref(K) if K else None, ARITH_FP32, None))
-            torch.cuda.synchronize()
-            out.append((screen, new))
-        assert_same_bits(out[0][0], out[1][0], "screen")
-        assert_same_bits(out[0][1], out[1][1], "history")
+        both_forms(w, U, W, H, W + pad, inputs(W, H, W, H, W + pad, W + pad, fmt, motion, odd, 71 + k), fmt, cas_for(w, W, H) if cas else None)
+
+
+# one row a thread below 800 regions (the first two sizes), two rows above; still texels are reprojected through the matrices
+@pytest.mark.parametrize("W,H,odd", [(95, 61, True), (3, 2, False), (1281, 721, True), (31, 24001, False)])
+def test_default_block_equals_the_general_form(W, H, odd):
+    for k, (cas, pad, reset, split) in enumerate([(True, 0, 0, 0), (False, 3, 0, 0), (True, 5, 0, W // 3), (True, 0, 1, 0)]):
+        print(f"case defaults {W}x{H} cas {cas} pad {pad} reset {reset} split {split}", flush=True)
+        w = workload("c2", fmt=FMT_RGBA16F, vel=VEL_RGBA16F)
+        U = uniforms_for(w, 1, (0.3 / W, -0.4 / H), params=default_params())
+        U.mHistoryViewProjMatrix[12], U.mHistoryViewProjMatrix[5], U.mHistoryViewProjMatrix[11] = 0.01, 0.98, 0.02
+        U.mResetHistory, U.splitScreen, U.splitX = reset, int(split > 0), split
+        color, depth, vel, hist, prev = inputs(W, H, W, H, W + pad, W + pad, FMT_RGBA16F, 5, odd, 91 + k)
+        moving = (torch.arange(W + pad, device="cuda") // 7 % 3 > 0).to(vel.dtype).expand(H, -1)
+        vel4 = torch.stack([vel[..., 0], vel[..., 1], torch.full_like(moving, 0.001), moving], -1).contiguous()
+        both_forms(w, U, W, H, W + pad, (color, depth, vel4, hist, prev), FMT_RGBA16F, cas_for(w, W, H) if cas else None)
 
 
 @pytest.mark.parametrize("specs", [[((480, 270), (480, 270)), ((640, 361), (640, 361)), ((33, 65), (33, 65))],
@@ -57,3 +76,13 @@ def test_equals_the_general_form(W, H, motion, odd, fmt):
 @pytest.mark.parametrize("fmt", [FMT_RGBA16F, FMT_RGBA32F])
 def test_batches(specs, fmt):
     batches(specs, fmt, ARITH_FP32)
+
+
+@pytest.mark.parametrize("specs", [[((480, 270), (480, 270)), ((33, 65), (33, 65))], [((960, 541), (960, 541)), ((640, 361), (640, 361))]])
+def test_default_block_batches(specs, monkeypatch):
+    import test_gpu_upscale as t
+    rgba = lambda *a, **k: (lambda i: (i[0], i[1], torch.cat([i[2], i[2].abs() * 50], -1).contiguous(), i[3], i[4]))(inputs(*a, **k))
+    monkeypatch.setattr(t, "inputs", rgba)
+    monkeypatch.setattr(t, "VEL_RG16F", VEL_RGBA16F)
+    monkeypatch.setattr(t, "uniforms_for", lambda w, f, j: uniforms_for(w, f, j, params=default_params()))
+    batches(specs, FMT_RGBA16F, ARITH_FP32)
