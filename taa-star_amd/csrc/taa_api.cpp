@@ -218,7 +218,8 @@ int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, in
         fd.x_end = x_end;
         fd.param_idx = param_idx;
         if (U.mUpsampling) fd.up = 1;
-        const int e = taastar::launch_resolve_seg(fd, U, *sg, arith, stream);
+        const int e = taastar::mask_form(fd, U) ? taastar::launch_mask(fd, U, *sg, arith, stream)
+                                                : taastar::launch_resolve_seg(fd, U, *sg, arith, stream);
         if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
         return TAA_OK;
     }

@@ -184,6 +184,11 @@ constexpr int kProdWindowCols = 48, kProdWindowRows = 12;  // the history window
 // general kernel's small tiles keep shorter.
 int launch_exact(const FrameDesc& fd, const taa_uniforms_t& U, void* stream);
 int launch_exact_batch(const BatchEntry* d_entries, int n_entries, int total, bool cas, bool s16, void* stream);
+// The masked resolve with the production feature set at one size, exact or FP16 arithmetic, and whether it takes a frame: from 700
+// workgroups (us, k_resolve_seg and this one, with CAS: FP32 storage 640x360 (572) 16.4 and 15.7, 320x180 7.9 and 11.2, FP16
+// storage and arithmetic 640x360 11.3 and 13.0, 1280x720 33 and 25; without CAS FP32 640x360 (460) 13.6 and 14.5, 1280x720 44 and 34).
+bool mask_form(const FrameDesc& fd, const taa_uniforms_t& U);
+int launch_mask(const FrameDesc& fd, const taa_uniforms_t& U, const SegDesc& sg, int arith, void* stream);
 inline long long exact_workgroups(bool cas, bool s16) { return cas || s16 ? 900 : 1500; }
 // The upsampling resolve, inputs no larger than the output.
 // LDS of a tile over a w x h rectangle of input texels, in front of the rectangle's boxes (24 bytes each): the staged

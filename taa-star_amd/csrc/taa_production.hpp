@@ -36,7 +36,7 @@ struct ProdGeo {
 // a resolve texel between its history position and its blend
 struct ProdTexel {
     float fx, fy, expected, pd, hu, hv;
-    bool outside;
+    bool outside, masked;  // masked: rejected by the segmentation mask
     int kx, ky, k;
 };
 
@@ -74,6 +74,18 @@ __device__ __forceinline__ f3 sqrt3(f3 v) {
     auto bits = [](float x) { return __float_as_uint(x) - 1u; };  // zero last
     if (min(min(bits(v.x), bits(v.y)), bits(v.z)) < __float_as_uint(0x1p-96f) - 1u) return {sqrtf(v.x), sqrtf(v.y), sqrtf(v.z)};
     return {root(v.x), root(v.y), root(v.z)};
+}
+
+// clip centre and half size of the FP16 path's box (clip_aabb_fast) from the 3x3 sums and sums of squares
+__device__ __forceinline__ void fast_box(f3 m1, f3 m2, float gamma, f3& c, f3& e) {
+    constexpr float inv9 = 1.0f / 9.0f;
+    const f3 mean = m1 * inv9;
+    const f3 sigma = {sqrt_fast(fmaxf(__builtin_fmaf(-mean.x, mean.x, m2.x * inv9), 0.0f)), sqrt_fast(fmaxf(__builtin_fmaf(-mean.y, mean.y, m2.y * inv9), 0.0f)),
+                      sqrt_fast(fmaxf(__builtin_fmaf(-mean.z, mean.z, m2.z * inv9), 0.0f))};
+    const f3 mn = {__builtin_fmaf(-gamma, sigma.x, mean.x), __builtin_fmaf(-gamma, sigma.y, mean.y), __builtin_fmaf(-gamma, sigma.z, mean.z)};
+    const f3 mx = {__builtin_fmaf(gamma, sigma.x, mean.x), __builtin_fmaf(gamma, sigma.y, mean.y), __builtin_fmaf(gamma, sigma.z, mean.z)};
+    c = {0.5f * (mx.x + mn.x), 0.5f * (mx.y + mn.y), 0.5f * (mx.z + mn.z)};
+    e = {__builtin_fmaf(0.5f, mx.x - mn.x, 1e-7f), __builtin_fmaf(0.5f, mx.y - mn.y, 1e-7f), __builtin_fmaf(0.5f, mx.z - mn.z, 1e-7f)};
 }
 
 // history position of a texel: base texel and fraction (taa.comp:456-462), the base widening the bounds of the thread's
@@ -286,7 +298,7 @@ __device__ __forceinline__ void finish(const FrameDesc& fd, const taa_uniforms_t
         }
         f3 hc = rgb_to_ycocg(acc);
         // rejection (taa.comp:787-823)
-        bool rejected = p.outside;
+        bool rejected = p.outside || p.masked;
         if (lin_thr > 0.0f ? linear_depth_reject(p.pd, p.expected, near, far, lin_thr) : fabsf(p.pd - p.expected) > 0.1f * (1.0f - p.pd)) rejected = true;
         // clipAabb (taa.comp:323-345) towards the box's centre c, half size e
         f3 cur;

@@ -167,15 +167,7 @@ __device__ __forceinline__ void resolve_upscale(const FrameDesc& fd, const taa_u
                     m1 = m1 + c[k];
                     m2 = {__builtin_fmaf(c[k].x, c[k].x, m2.x), __builtin_fmaf(c[k].y, c[k].y, m2.y), __builtin_fmaf(c[k].z, c[k].z, m2.z)};
                 }
-                constexpr float inv9 = 1.0f / 9.0f;
-                const f3 mean = m1 * inv9;
-                const f3 sigma = {sqrt_fast(fmaxf(__builtin_fmaf(-mean.x, mean.x, m2.x * inv9), 0.0f)),
-                                  sqrt_fast(fmaxf(__builtin_fmaf(-mean.y, mean.y, m2.y * inv9), 0.0f)),
-                                  sqrt_fast(fmaxf(__builtin_fmaf(-mean.z, mean.z, m2.z * inv9), 0.0f))};
-                const f3 mn = {__builtin_fmaf(-gamma, sigma.x, mean.x), __builtin_fmaf(-gamma, sigma.y, mean.y), __builtin_fmaf(-gamma, sigma.z, mean.z)};
-                const f3 mx = {__builtin_fmaf(gamma, sigma.x, mean.x), __builtin_fmaf(gamma, sigma.y, mean.y), __builtin_fmaf(gamma, sigma.z, mean.z)};
-                p = {0.5f * (mx.x + mn.x), 0.5f * (mx.y + mn.y), 0.5f * (mx.z + mn.z)};  // clip_aabb_fast's centre and half size
-                e = {__builtin_fmaf(0.5f, mx.x - mn.x, 1e-7f), __builtin_fmaf(0.5f, mx.y - mn.y, 1e-7f), __builtin_fmaf(0.5f, mx.z - mn.z, 1e-7f)};
+                fast_box(m1, m2, gamma, p, e);
             } else {
                 f3 m1 = c[0] + c[1] + c[2] + c[3] + c[4] + c[5] + c[6] + c[7] + c[8];
                 f3 m2 = c[0] * c[0] + c[1] * c[1] + c[2] * c[2] + c[3] * c[3] + c[4] * c[4] + c[5] * c[5] + c[6] * c[6] + c[7] * c[7] + c[8] * c[8];
@@ -241,6 +233,7 @@ __device__ __forceinline__ void resolve_upscale(const FrameDesc& fd, const taa_u
             q[k].expected = sd[l];
             q[k].hu = hu;
             q[k].hv = hv;
+            q[k].masked = false;
             // the previous depth under the history position (taa.comp:818)
             q[k].pd = __uint_as_float(hdepth.ld1(((uint32_t)med3<0>(to_int(hv * fHl), Hl - 1) * pl + (uint32_t)med3<0>(to_int(hu * fWl), Wl - 1)) * 4u, 0u));
             // current colour: the texel itself, or getCurrentUpsampledColor's (taa.comp:222-257, 750-755)

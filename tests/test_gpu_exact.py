@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 
 from gpu_helpers import assert_same_bits  # noqa: E402
 from test_gpu_upscale import inputs, test_batches_equal_sessions_alone as batches  # noqa: E402
-from taastar import (ARITH_FP32, FMT_RGBA16F, FMT_RGBA32F, VEL_RG16F, VEL_RG32F, VEL_RGBA16F, FrameImages, check,  # noqa: E402
-                     default_params, lib)
+from taastar import (ARITH_FP16, ARITH_FP32, FMT_RGBA16F, FMT_RGBA32F, RTFLAG, VEL_RG16F, VEL_RG32F, VEL_RGBA16F, FrameImages,  # noqa: E402
+                     SegmentationImages, check, default_params, lib)
 from taastar.workloads import cas_for, uniforms_for, workload  # noqa: E402
 
 
@@ -21,8 +21,8 @@ def _need_gpu():
         pytest.skip("no GPU")
 
 
-def both_forms(w, U, W, H, pitch, images, fmt, K):
-    """Screen and history of the frame without and with a debug image."""
+def both_forms(w, U, W, H, pitch, images, fmt, K, arith=ARITH_FP32, seg=None):
+    """Screen and history of the frame without and with a debug image; seg: the mask's images, its output too."""
     color, depth, vel, hist, prev = images
     out = []
     for general in (False, True):
@@ -35,9 +35,17 @@ def both_forms(w, U, W, H, pitch, images, fmt, K):
         img.debug = debug.data_ptr() if general else None
         img.width, img.height, img.pitch = W, H, pitch
         img.color_format, img.velocity_format = fmt, w["vel"]
-        check(lib().taa_resolve_frame(C.byref(U), C.byref(img), C.byref(K) if K else None, ARITH_FP32, None))
+        mask = torch.full((H, pitch), 7, dtype=torch.int32, device="cuda")
+        if seg is None:
+            check(lib().taa_resolve_frame(C.byref(U), C.byref(img), C.byref(K) if K else None, arith, None))
+        else:
+            g = SegmentationImages()
+            g.material, g.prev_material, g.uv_normal, g.prev_segmask = [t.data_ptr() for t in seg]
+            g.segmask, g.pitch, g.input_pitch = mask.data_ptr(), pitch, seg[0].shape[1]
+            check(lib().taa_resolve_frame_segmented(C.byref(U), C.byref(img), C.byref(g), C.byref(K) if K else None, arith, None))
         torch.cuda.synchronize()
-        out.append((screen, new))
+        out.append((screen, new, mask))
+    assert torch.equal(out[0][2], out[1][2]), "mask"
     assert_same_bits(out[0][0], out[1][0], "screen")
     assert_same_bits(out[0][1], out[1][1], "history")
 
@@ -86,3 +94,32 @@ def test_default_block_batches(specs, monkeypatch):
     monkeypatch.setattr(t, "VEL_RG16F", VEL_RGBA16F)
     monkeypatch.setattr(t, "uniforms_for", lambda w, f, j: uniforms_for(w, f, j, params=default_params()))
     batches(specs, FMT_RGBA16F, ARITH_FP32)
+
+
+F = RTFLAG
+FLAGS = [F["OUT"] | F["DIS"] | F["NRM"] | F["DPT"] | F["MID"] | F["LUM"] | F["CNT"], F["DPT"] | F["LUM"], F["OUT"] | F["DIS"] | F["MID"],
+         F["NRM"] | F["CNT"] | F["FXD"], F["ALL"], F["ALL"] | F["FXD"] | F["OUT"] | F["DIS"], 0]
+
+
+# 700 regions select the kernel: one region wide and high, inner tiles beyond the 100-texel border of FXD, and below the line
+@pytest.mark.parametrize("W,H,odd", [(5, 12001, True), (22801, 7, False), (1021, 701, True), (61, 29, False)])
+@pytest.mark.parametrize("fmt,arith", [(FMT_RGBA16F, ARITH_FP16), (FMT_RGBA16F, ARITH_FP32), (FMT_RGBA32F, ARITH_FP16), (FMT_RGBA32F, ARITH_FP32)])
+def test_mask_equals_the_general_form(W, H, odd, fmt, arith):
+    for k, flags in enumerate(FLAGS):
+        cas, pad, split = k % 3 != 1, k % 2 * 3, W // 3 if k == 3 else 0
+        print(f"case mask {W}x{H} fmt {fmt} arith {arith} flags {flags:#x} cas {cas} pad {pad} split {split}", flush=True)
+        w = workload("c2", fmt=fmt, vel=VEL_RG16F if fmt == FMT_RGBA16F else VEL_RG32F)
+        p = w["params"]()
+        p.mRayTraceAugment, p.mRayTraceAugmentFlags, p.mRayTraceHistoryCount = 1, flags, 4
+        U = uniforms_for(w, 1, (0.3 / W, -0.4 / H), params=p)
+        U.splitScreen, U.splitX = int(split > 0), split
+        pitch, spl = W + pad, W + 2 * pad
+        images = inputs(W, H, W, H, pitch, pitch, fmt, 4, odd, 131 + k)
+        g = torch.Generator(device="cuda").manual_seed(k)
+        cells = torch.randint(0, 5, ((H + 4) // 5, (spl + 6) // 7), generator=g, device="cuda").repeat_interleave(5, 0).repeat_interleave(7, 1)[:H, :spl]
+        moved = torch.rand(H, spl, generator=g, device="cuda") < 0.05
+        material = cells.to(torch.int32).contiguous()
+        prev = torch.where(moved, cells + 1, cells).to(torch.int32) | torch.where(cells % 2 == 0, -2**31, 0).to(torch.int32)
+        normals = (cells[..., None].float() + 0.2 * torch.rand(H, spl, 4, generator=g, device="cuda")).contiguous()
+        old = torch.where(torch.rand(H, pitch, generator=g, device="cuda") < 0.1, (3 << 16) | 2, 0).to(torch.int32)
+        both_forms(w, U, W, H, pitch, images, fmt, cas_for(w, W, H) if cas else None, arith, (material, prev.contiguous(), normals, old))
