@@ -35,7 +35,7 @@ SOURCES = [
     ("taa_upscale.hip", "hip"),
     ("taa_exact.hip", "hip"),
     ("taa_velocity.hip", "hip"),
-    ("taa_edge_aa.hip", "hip"),
+    ("taa_post.hip", "hip"),
     ("taa_noalloc.hip", "hip"),
     ("taa_api.cpp", "cxx"),
     ("taa_host.cpp", "cxx"),

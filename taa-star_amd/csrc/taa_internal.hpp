@@ -100,7 +100,6 @@ int launch_resolve_up(const FrameDesc& fd, const taa_uniforms_t& U, int arith, v
 // where no selection depends on it); fd.up: the upsampling path's kernel, which reads the mask's
 // inputs from global memory. Tiled by its own shape, whatever fd.tiles_x / tiles_y say
 int launch_resolve_seg(const FrameDesc& fd, const taa_uniforms_t& U, const SegDesc& sg, int arith, void* stream);
-int launch_cas(const void* src, void* dst, int W, int H, int pitch, int fmt, uint32_t peak_bits, void* stream);
 // Workgroups of a batched launch: one per tile, rounded to whole XCD slots; the batch kernels take
 // exactly this grid and resolve one tile per workgroup (batch_tile). Measured on the 64-session
 // mix, one workgroup per tile with the hardware dispatcher balancing the XCDs is faster (55.7 vs
@@ -219,9 +218,11 @@ int upscale_variant(long long n16, long long n32, int lds);
 int launch_upscale(const FrameDesc& fd, const taa_uniforms_t& U, int arith, void* stream);
 int launch_upscale_batch(const BatchEntry* d_entries, int n_entries, int total, int variant, int lds, bool cas, bool s16, int arith, void* stream);
 
-// Edge-AA fallback on category-1 texels of a segmentation mask (taa_edge_aa.hip).
+// Edge-AA fallback on category-1 texels of a segmentation mask (taa_post.hip).
 int launch_edge_aa(const void* src, const uint32_t* mask, void* dst, int W, int H, int pitch, int seg_pitch, int fmt,
                    float subpix, float thr, float thr_min, void* stream);
+// sharpen_cas.comp on its own (taa_post.hip).
+int launch_cas(const void* src, void* dst, int W, int H, int pitch, int fmt, uint32_t peak_bits, void* stream);
 
 // TAA_OK, or the status taa_batch_submit returns for a frame with these uniforms (taa_api.cpp).
 int check_batch_uniforms(const taa_uniforms_t* u);

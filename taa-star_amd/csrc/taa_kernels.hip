@@ -1044,18 +1044,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FA && S16 ?
     resolve_tile<G, S16, false, FA, PROD>(e.fd, e.U, t - e.tile_begin, sm);
 }
 
-// sharpen_cas.comp on its own (one thread per pixel, clamped loads)
-template <bool S16>
-__global__ __launch_bounds__(256) void k_cas(const void* __restrict__ src, void* __restrict__ dst, int W, int H, int pitch, uint32_t peak_bits) {
-    const int x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 16 + (threadIdx.x >> 4);
-    if (x >= W || y >= H) return;
-    auto ld = [&](int xx, int yy) {
-        return xyz(ld_rgba<S16>(src, (uint32_t)(clampi(yy, 0, H - 1) * pitch + clampi(xx, 0, W - 1))));
-    };
-    f3 o = cas_filter(ld(x, y - 1), ld(x - 1, y), ld(x, y), ld(x + 1, y), ld(x, y + 1), __uint_as_float(peak_bits));
-    st_rgba<S16>(dst, (uint32_t)(y * pitch + x), make_float4(o.x, o.y, o.z, 1.0f));
-}
-
 // ------------------------------------------------------------------------------------------
 // dispatch tables
 
@@ -1194,14 +1182,6 @@ int launch_resolve_seg(const FrameDesc& fd, const taa_uniforms_t& U, const SegDe
     if (fd.up) e = fa ? launch_resolve_seg_t<true, true>(a, sg, st) : launch_resolve_seg_t<true, false>(a, sg, st);
     else e = fa ? launch_resolve_seg_t<false, true>(a, sg, st) : launch_resolve_seg_t<false, false>(a, sg, st);
     return (int)e;
-}
-
-int launch_cas(const void* src, void* dst, int W, int H, int pitch, int fmt, uint32_t peak_bits, void* stream) {
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    dim3 grid((W + 15) / 16, (H + 15) / 16);
-    if (fmt == TAA_FMT_RGBA16F) hipLaunchKernelGGL(k_cas<true>, grid, dim3(256), 0, st, src, dst, W, H, pitch, peak_bits);
-    else hipLaunchKernelGGL(k_cas<false>, grid, dim3(256), 0, st, src, dst, W, H, pitch, peak_bits);
-    return (int)hipGetLastError();
 }
 
 template <bool FA, bool PROD>
