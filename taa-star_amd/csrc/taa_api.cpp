@@ -256,10 +256,13 @@ int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, in
     } else {
         taastar::FrameDesc p = fd;
         taastar::tile_production(p, taastar::kProd256x2);
-        if (taastar::exact_prod_form(fd, U) &&
-            (long long)p.tiles_x * p.tiles_y >= taastar::exact_workgroups(cas, fd.color_fmt == TAA_FMT_RGBA16F))
-            e = taastar::launch_exact(p, U, stream);
-        else
+        const long long n16 = (long long)p.tiles_x * p.tiles_y;
+        if (taastar::exact_prod_form(fd, U) && n16 >= taastar::exact_workgroups(cas, fd.color_fmt == TAA_FMT_RGBA16F)) {
+            e = taastar::launch_exact(p, U, false, stream);
+        } else if (taastar::exact_plain_form(fd, U)) {
+            taastar::tile_production(p, taastar::plain_variant(n16, cas));
+            e = taastar::launch_exact(p, U, true, stream);
+        } else
             e = taastar::launch_resolve(fd, U, shape, arith, stream);
     }
     if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
@@ -847,6 +850,7 @@ struct BatchLayout {
     int form = 0;  // the FP16 kernel's form (taastar::fast_path_form): the largest over the frames
     bool prod_main = false, prod_up = false;  // every frame of that launch has the production feature set
     bool exact = false;  // the one-size frames take the exact kernel of taa_exact.hip
+    bool plain = false;  // ... in its plain form
     int n_main = 0, total_main = 0;
     int n_up = 0, total_up = 0;
     int up_variant = 0, up_lds = 0;  // every upsampling frame takes the kernel of taa_upscale.hip: its variant and LDS
@@ -957,14 +961,16 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
     for (int i = 0; i < L.n_main && L.prod_main; ++i) L.prod_main = taastar::exact_prod_form(ents[i].fd, ents[i].U);
     L.prod_up = L.n_up > 0;
     for (int i = L.n_main; i < L.n_main + L.n_up && L.prod_up; ++i) L.prod_up = taastar::prod_params(ents[i].fd, ents[i].U);
-    if (L.prod_main) {
+    L.plain = !L.fast && !L.window && L.n_main > 0;
+    for (int i = 0; i < L.n_main && L.plain; ++i) L.plain = taastar::exact_plain_form(ents[i].fd, ents[i].U);
+    if (L.prod_main || L.plain) {
         long long n16 = 0;
         for (int i = 0; i < L.n_main; ++i) {
             taastar::FrameDesc fd = ents[i].fd;
             taastar::tile_production(fd, taastar::kProd256x2);
             n16 += (long long)fd.tiles_x * fd.tiles_y;
         }
-        L.exact = n16 >= taastar::exact_workgroups(L.cas, L.s16);
+        L.exact = L.plain || n16 >= taastar::exact_workgroups(L.cas, L.s16);
         if (L.exact) L.total_main = 0;
         for (int i = 0; i < L.n_main && L.exact; ++i) {
             taastar::BatchEntry& e = ents[i];
@@ -1015,7 +1021,7 @@ static int build_batch(taa_ctx_t* c, int n, const taa_batch_item_t* items, int a
 static int launch_layout(const taastar::BatchEntry* d_ents, const BatchLayout& L, int arith, void* stream) {
     if (L.n_main) {
         int le = L.window ? taastar::launch_window_batch(d_ents, L.n_main, L.total_main, L.rows, L.cas, L.form, stream)
-                 : L.exact ? taastar::launch_exact_batch(d_ents, L.n_main, L.total_main, L.cas, L.s16, stream)
+                 : L.exact ? taastar::launch_exact_batch(d_ents, L.n_main, L.total_main, L.plain, L.cas, L.s16, stream)
                  : L.fast ? taastar::launch_batch_fast(d_ents, L.n_main, L.total_main, L.shape, L.cas, L.form, stream)
                         : taastar::launch_batch(d_ents, L.n_main, L.total_main, L.shape, L.cas, L.s16, arith, L.prod_main,
                                                 stream);
@@ -1093,7 +1099,7 @@ void plan_free(taa_batch_plan* p) {
 }
 
 bool same_launches(const BatchLayout& a, const BatchLayout& b) {
-    return a.shape == b.shape && a.fast == b.fast && a.window == b.window && a.rows == b.rows && a.form == b.form && a.prod_main == b.prod_main && a.exact == b.exact &&
+    return a.shape == b.shape && a.fast == b.fast && a.window == b.window && a.rows == b.rows && a.form == b.form && a.prod_main == b.prod_main && a.exact == b.exact && a.plain == b.plain &&
            a.prod_up == b.prod_up && a.n_main == b.n_main &&
            a.total_main == b.total_main &&
            a.n_up == b.n_up && a.total_up == b.total_up && a.up_variant == b.up_variant && a.up_lds == b.up_lds;

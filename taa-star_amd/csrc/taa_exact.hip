@@ -15,6 +15,8 @@
 // us a frame, before and now: with the mask 1920x1080 FP32 storage with CAS 115 and 72.6, FP16 storage and arithmetic 82 and
 // 53; without it FP32 storage with CAS 1920x1080 58.6 and 49.0, 3840x2160 208 and 203, without CAS 1920x1080
 // 52.7 and 42.0, 3840x2160 200 and 168; FP16 storage with CAS 1920x1080 54.2 and 42.8, 3840x2160 186 and 169.
+// The plain form (no closest-depth velocity, depth culling, Lottes weighting or outside rejection) ran the general kernel with its
+// switches: FP32 storage 640x360 without CAS 10.5 and 7.8, 1920x1080 with CAS 77 and 44, FP16 storage 68 and 38.
 // Measured and not kept: four rows a thread (1920x1080 with CAS 51.6, 3840x2160 211: four waves a SIMD), 512 threads of two
 // rows (55.7, 235) or of one (54.6; footprints gathered without the window 65.8).
 #include <hip/hip_runtime.h>
@@ -29,16 +31,18 @@
 namespace taastar {
 namespace {
 
-// SEG: the frame also writes the segmentation mask
-template <bool CAS, bool S16, bool SEG_ = false, bool FA = false>
-struct ExactGeo : ProdGeo<256, 2, CAS, S16, FA> {
-    typedef ProdGeo<256, 2, CAS, S16, FA> Base;
-    static constexpr bool SEG = SEG_;
+// SEG: the frame also writes the segmentation mask; PLAIN: the texel's own velocity, no depth culling, Lottes weighting or
+// outside rejection
+template <bool CAS, bool S16, bool SEG_ = false, bool FA = false, bool PLAIN_ = false, int NT = 256, int RPT = 2>
+struct ExactGeo : ProdGeo<NT, RPT, CAS, S16, FA> {
+    typedef ProdGeo<NT, RPT, CAS, S16, FA> Base;
+    static constexpr bool SEG = SEG_, PLAIN = PLAIN_;
     typedef typename Base::VelT VelT;
-    static constexpr int RW = Base::RW, RH = Base::RH, NT = Base::NT;
+    static constexpr int RW = Base::RW, RH = Base::RH;
     // staged inputs: the region and one texel around it, two texels of a row a thread, SR rows a pass
     static constexpr int SW = RW + 2, SH = RH + 2, NS = SW * SH, SC = SW / 2, SR = NT / SC, SP = (SH + SR - 1) / SR;
-    static constexpr int kStaged = NS * (4 + (int)sizeof(VelT) + (SEG ? 20 : 0)), kWin = Base::WP * Base::WH * (int)sizeof(typename Base::Win),
+    static constexpr int kStaged = PLAIN ? 0 : NS * (4 + (int)sizeof(VelT) + (SEG ? 20 : 0)),
+                         kWin = Base::WIN ? Base::WP * Base::WH * (int)sizeof(typename Base::Win) : 16,
                          kRes = RW * RH * Base::TB, kMost = kStaged > kWin ? kStaged : kWin;
     struct Smem {
         alignas(16) unsigned char win[kMost > kRes ? kMost : kRes];  // velocity, depth and the mask's inputs, then the window, then the resolved texels
@@ -74,12 +78,27 @@ __device__ __forceinline__ void resolve_exact(const FrameDesc& fd, const taa_uni
         normals(SEG ? (const void*)sg->uv_normal : nullptr, SEG ? sg->pitch_l : 1, SEG ? W : 1, SEG ? H : 1, 16),
         prev_materials(SEG ? (const void*)sg->prev_material : nullptr, SEG ? sg->pitch_l : 1, SEG ? W : 1, SEG ? H : 1, 4);
 
+    float2 own[G::PLAIN ? RPT : 1];  // the thread's texels' velocities
+    if constexpr (G::PLAIN) {
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            const uint32_t i = (uint32_t)clampi(y0 + rg + k, 0, H - 1) * pitch + (uint32_t)clampi(x0 + rx, 0, W - 1);
+            if constexpr (S16) {
+                own[k] = vel_xy(velocity.ld1(i * 4u, 0u));
+            } else {
+                const uint2 v = velocity.ld2(i * 8u, 0u);
+                own[k] = make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
+            }
+        }
+    }
+
     // ---- 1. stage colour, depth and velocity of the region and one texel around it, clamped to the edge
     {
         auto store = [&](int i, f3 a, f3 b, uint2 d, VelT v0, VelT v1) {
             a = rgb_to_ycocg(a), b = rgb_to_ycocg(b);
             *reinterpret_cast<float4*>(sm.c01 + i) = make_float4(a.x, a.y, b.x, b.y);
             *reinterpret_cast<float2*>(sm.c2 + i) = make_float2(a.z, b.z);
+            if constexpr (G::PLAIN) return;
             *reinterpret_cast<uint2*>(sd + i) = d;
             sv[i] = v0;
             sv[i + 1] = v1;
@@ -174,7 +193,18 @@ __device__ __forceinline__ void resolve_exact(const FrameDesc& fd, const taa_uni
     // ---- 2. closest depth, history position and previous depth of the thread's texels
     ProdTexel q[RPT];
     int4 bases = make_int4(0x7fffffff, 0x7fffffff, 0x7fffffff, 0x7fffffff);
-    {
+    if constexpr (G::PLAIN) {  // SAMPLE_TEX(uCurrentVelocity, uv) (taa.comp:421)
+        const float uvx = sm.ux[rx + 1];
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            const float2 v = own[k];
+            q[k].expected = q[k].pd = 0.0f;
+            q[k].hu = uvx - v.x;
+            q[k].hv = sm.uy[rg + k + 1] - v.y;
+            q[k].masked = false;
+            history_base<FA>(q[k], W, H, bases);
+        }
+    } else {
         const int base = rg * SW + rx;
         struct Row {
             float d, cd;  // the first smallest depth of the row's three in scan order (strict <), the centre's
@@ -317,24 +347,33 @@ struct ResolveArgs {
     taa_uniforms_t U;
 };
 
-constexpr int exact_waves(bool s16) { return s16 ? 6 : 5; }  // occupancy hint (waves per SIMD): what the LDS of the tile allows
+// occupancy hint (waves per SIMD): what the LDS of the tile allows
+template <class G>
+constexpr int exact_waves() {
+    return G::RPT == 1 ? 4 : G::S16 ? 6 : 5;
+}
 
-template <bool CAS, bool S16>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(exact_waves(S16)))) void k_resolve_exact(const ResolveArgs a) {
-    using G = ExactGeo<CAS, S16>;
+template <class G>
+__global__ __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(exact_waves<G>()))) void k_resolve_exact(const ResolveArgs a) {
     __shared__ typename G::Smem sm;
     resolve_exact<G>(a.fd, a.U, xcd_tile((int)blockIdx.x, a.fd.tiles_x * a.fd.tiles_y), sm);
 }
 
 // the frames of a batch, walked like the other batched kernels
-template <bool CAS, bool S16>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(exact_waves(S16)))) void k_resolve_exact_batch(const BatchEntry* __restrict__ entries, int n_entries, int total) {
-    using G = ExactGeo<CAS, S16>;
+template <class G>
+__global__ __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(exact_waves<G>()))) void k_resolve_exact_batch(const BatchEntry* __restrict__ entries, int n_entries, int total) {
     __shared__ typename G::Smem sm;
     const int t = batch_tile(total);
     if (t < 0) return;
     const BatchEntry& e = batch_entry(entries, n_entries, t);
     resolve_exact<G>(e.fd, e.U, t - e.tile_begin, sm);
+}
+
+// f(geometry) for a frame's form
+template <bool PLAIN, int NT, int RPT, class F>
+void for_form(bool cas, bool s16, F&& f) {
+    if (cas) s16 ? f(ExactGeo<true, true, false, false, PLAIN, NT, RPT>()) : f(ExactGeo<true, false, false, false, PLAIN, NT, RPT>());
+    else s16 ? f(ExactGeo<false, true, false, false, PLAIN, NT, RPT>()) : f(ExactGeo<false, false, false, false, PLAIN, NT, RPT>());
 }
 
 // the resolve with the segmentation mask of mRayTraceAugment (FA: the FP16 path's arithmetic where no selection depends on it)
@@ -377,33 +416,29 @@ int launch_mask(const FrameDesc& fd, const taa_uniforms_t& U, const SegDesc& sg,
     return (int)hipGetLastError();
 }
 
-int launch_exact(const FrameDesc& fd, const taa_uniforms_t& U, void* stream) {
+int launch_exact(const FrameDesc& fd, const taa_uniforms_t& U, bool plain, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     ResolveArgs a;
     a.fd = fd;
     a.U = U;
-    const dim3 g(fd.tiles_x * fd.tiles_y);
-    const bool s16 = fd.color_fmt == TAA_FMT_RGBA16F;
-    if (fd.cas_on) {
-        if (s16) hipLaunchKernelGGL((k_resolve_exact<true, true>), g, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_resolve_exact<true, false>), g, dim3(256), 0, st, a);
-    } else {
-        if (s16) hipLaunchKernelGGL((k_resolve_exact<false, true>), g, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_resolve_exact<false, false>), g, dim3(256), 0, st, a);
-    }
+    const bool cas = fd.cas_on != 0, s16 = fd.color_fmt == TAA_FMT_RGBA16F;
+    auto launch = [&](auto g) {
+        hipLaunchKernelGGL((k_resolve_exact<decltype(g)>), dim3(fd.tiles_x * fd.tiles_y), dim3(decltype(g)::NT), 0, st, a);
+    };
+    if (!plain) for_form<false, 256, 2>(cas, s16, launch);
+    else if (fd.rows != kProd512x1) for_form<true, 256, 2>(cas, s16, launch);
+    else if (s16) launch(ExactGeo<false, true, false, false, true, 512, 1>());  // (chosen without CAS only)
+    else launch(ExactGeo<false, false, false, false, true, 512, 1>());
     return (int)hipGetLastError();
 }
 
-int launch_exact_batch(const BatchEntry* e, int n, int total, bool cas, bool s16, void* stream) {
+int launch_exact_batch(const BatchEntry* e, int n, int total, bool plain, bool cas, bool s16, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 g(batch_grid(total));
-    if (cas) {
-        if (s16) hipLaunchKernelGGL((k_resolve_exact_batch<true, true>), g, dim3(256), 0, st, e, n, total);
-        else hipLaunchKernelGGL((k_resolve_exact_batch<true, false>), g, dim3(256), 0, st, e, n, total);
-    } else {
-        if (s16) hipLaunchKernelGGL((k_resolve_exact_batch<false, true>), g, dim3(256), 0, st, e, n, total);
-        else hipLaunchKernelGGL((k_resolve_exact_batch<false, false>), g, dim3(256), 0, st, e, n, total);
-    }
+    auto launch = [&](auto g) {
+        hipLaunchKernelGGL((k_resolve_exact_batch<decltype(g)>), dim3(batch_grid(total)), dim3(256), 0, st, e, n, total);
+    };
+    if (plain) for_form<true, 256, 2>(cas, s16, launch);
+    else for_form<false, 256, 2>(cas, s16, launch);
     return (int)hipGetLastError();
 }
 

@@ -88,6 +88,9 @@ int launch_resolve(const FrameDesc& fd, const taa_uniforms_t& U, int shape, int 
 // culling, Lottes, outside rejection; no debug or inspect image): the general kernel's arithmetic
 // with the other branches compiled out
 bool exact_prod_form(const FrameDesc& fd, const taa_uniforms_t& U);
+// the same for its plain form: the production set without closest-depth velocity, depth culling, Lottes weighting and
+// outside rejection (each texel's own velocity, mAlpha)
+bool exact_plain_form(const FrameDesc& fd, const taa_uniforms_t& U);
 // the same switches, whatever the sizes: launch_upscale (or, for the sizes it does not take, launch_resolve_up's
 // production form) runs when they hold; with seg, the same with mRayTraceAugment set (the masked resolve's
 // production form, whose mask keeps its own parameters)
@@ -181,13 +184,16 @@ constexpr int kProdWindowCols = 48, kProdWindowRows = 12;  // the history window
 // 15.6, 18.9 and 15.1; without CAS FP32 960x540 (1020) 12.7 and 13.8, 1280x720 (1800) 19.6 and 19.6, FP16 640x360 (460) 7.8
 // and 8.1, 960x540 13.2 and 12.2): below, most of a workgroup's time is the chain of its loads and barriers, which the
 // general kernel's small tiles keep shorter.
-int launch_exact(const FrameDesc& fd, const taa_uniforms_t& U, void* stream);
-int launch_exact_batch(const BatchEntry* d_entries, int n_entries, int total, bool cas, bool s16, void* stream);
+int launch_exact(const FrameDesc& fd, const taa_uniforms_t& U, bool plain, void* stream);
+int launch_exact_batch(const BatchEntry* d_entries, int n_entries, int total, bool plain, bool cas, bool s16, void* stream);
 // The masked resolve with the production feature set at one size, exact or FP16 arithmetic, and whether it takes a frame: from 700
 // workgroups (us, k_resolve_seg and this one, with CAS: FP32 storage 640x360 (572) 16.4 and 15.7, 320x180 7.9 and 11.2, FP16
 // storage and arithmetic 640x360 11.3 and 13.0, 1280x720 33 and 25; without CAS FP32 640x360 (460) 13.6 and 14.5, 1280x720 44 and 34).
 bool mask_form(const FrameDesc& fd, const taa_uniforms_t& U);
 int launch_mask(const FrameDesc& fd, const taa_uniforms_t& U, const SegDesc& sg, int arith, void* stream);
+// The plain form is taken at every size (general kernel and this one, FP32 storage: 320x180 with CAS 7.8 and 7.0), without CAS on
+// kProd512x1 regions below 800 workgroups (640x360 7.8, two rows a thread 8.3; 960x540 (1020) 13.1 and 11.9).
+inline int plain_variant(long long n16, bool cas) { return !cas && n16 < 800 ? kProd512x1 : kProd256x2; }
 inline long long exact_workgroups(bool cas, bool s16) { return cas || s16 ? 900 : 1500; }
 // The upsampling resolve, inputs no larger than the output.
 // LDS of a tile over a w x h rectangle of input texels, in front of the rectangle's boxes (24 bytes each): the staged

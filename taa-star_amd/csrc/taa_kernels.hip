@@ -1078,20 +1078,32 @@ hipError_t launch_batch_t(const BatchEntry* e, int n, int total, int shape, hipS
 
 }  // namespace
 
-bool prod_params(const FrameDesc& fd, const taa_uniforms_t& U, bool seg) {
+namespace {
+// the switches that the production set and the plain form share
+bool common_params(const FrameDesc& fd, const taa_uniforms_t& U, bool seg) {
     const taa_params_t& p = U.param[fd.param_idx];
     const bool s16 = fd.color_fmt == TAA_FMT_RGBA16F;
     return !fd.debug && !fd.inspect && !U.mBypassHistoryUpdate &&
            fd.vel_fmt == (s16 ? TAA_VEL_RG16F : TAA_VEL_RG32F) && !p.mPassThrough && !p.mUnjitterNeighbourhood &&
            !p.mUnjitterCurrentSample && p.mVarianceClipping && !p.mShapedNeighbourhood && p.mUseYCoCg &&
-           !p.mShrinkChromaAxis && p.mUseVelocityVectors == 2 && p.mVelocitySampleMode == 2 && p.mDepthCulling &&
-           p.mInterpolationMode == 2 && !p.mDynamicAntiGhosting && (p.mRayTraceAugment != 0) == seg &&
-           p.mColorClampingOrClipping == 2 &&
-           !p.mVelBasedAlpha && p.mLumaWeightingLottes && !p.mReduceBlendNearClamp && p.mRejectOutside && !p.mAddNoise &&
-           !p.mToneMapLumaKaris;
+           !p.mShrinkChromaAxis && p.mUseVelocityVectors == 2 && p.mInterpolationMode == 2 && !p.mDynamicAntiGhosting &&
+           (p.mRayTraceAugment != 0) == seg && p.mColorClampingOrClipping == 2 && !p.mVelBasedAlpha &&
+           !p.mReduceBlendNearClamp && !p.mAddNoise && !p.mToneMapLumaKaris;
+}
+}  // namespace
+
+bool prod_params(const FrameDesc& fd, const taa_uniforms_t& U, bool seg) {
+    const taa_params_t& p = U.param[fd.param_idx];
+    return common_params(fd, U, seg) && p.mVelocitySampleMode == 2 && p.mDepthCulling && p.mLumaWeightingLottes && p.mRejectOutside;
 }
 
 bool exact_prod_form(const FrameDesc& fd, const taa_uniforms_t& U) { return !fd.up && !U.mUpsampling && prod_params(fd, U); }
+
+bool exact_plain_form(const FrameDesc& fd, const taa_uniforms_t& U) {
+    const taa_params_t& p = U.param[fd.param_idx];
+    return !fd.up && !U.mUpsampling && common_params(fd, U, false) && p.mVelocitySampleMode == 0 && !p.mDepthCulling &&
+           !p.mLumaWeightingLottes && !p.mRejectOutside;
+}
 
 int launch_resolve(const FrameDesc& fd, const taa_uniforms_t& U, int shape, int arith, void* stream) {
     (void)arith;

@@ -18,6 +18,7 @@ namespace {
 template <int NT_, int RPT_, bool CAS_, bool S16_, bool FA_>
 struct ProdGeo {
     static constexpr bool CAS = CAS_, S16 = S16_, FA = FA_;
+    static constexpr bool PLAIN = false;  // without depth culling, Lottes weighting and outside rejection
     static constexpr int NT = NT_, RPT = RPT_, RW = 32, RH = NT / 32 * RPT, RA = CAS ? 1 : 0, TW = RW - 2 * RA, TH = RH - 2 * RA;
     typedef typename std::conditional<S16, uint32_t, float2>::type VelT;  // staged velocity: the image's texel
     typedef typename std::conditional<S16, uint2, float4>::type Tex;      // a colour texel; a resolved texel for the CAS
@@ -139,7 +140,7 @@ __device__ __forceinline__ void finish(const FrameDesc& fd, const taa_uniforms_t
     if constexpr (!G::WIN) {
 #pragma unroll
         for (int k = 0; k < RPT; ++k) {
-            q[k].outside = q[k].hu < 0.0f || q[k].hv < 0.0f || q[k].hu >= 1.0f || q[k].hv >= 1.0f;
+            q[k].outside = !G::PLAIN && (q[k].hu < 0.0f || q[k].hv < 0.0f || q[k].hu >= 1.0f || q[k].hv >= 1.0f);
             // from a base that keeps the footprint inside the image; a wave with one over its edge (or an image too small) reads
             // the texels one by one, clamped
             const int kx = q[k].kx - 1, ky = q[k].ky - 1, bx = max(min(kx, W - 4), 0), by = max(min(ky, H - 4), 0);
@@ -177,7 +178,7 @@ __device__ __forceinline__ void finish(const FrameDesc& fd, const taa_uniforms_t
 #pragma unroll
         for (int k = 0; k < RPT; ++k) q[k].outside = false;
         // positions outside the image: none in a wave whose bases all lie in 0 .. size - 2
-        if (wb.x < 0 || wb.y < 0 || wb.z < 2 - W || wb.w < 2 - H) {
+        if (!G::PLAIN && (wb.x < 0 || wb.y < 0 || wb.z < 2 - W || wb.w < 2 - H)) {
 #pragma unroll
             for (int k = 0; k < RPT; ++k) q[k].outside = q[k].hu < 0.0f || q[k].hv < 0.0f || q[k].hu >= 1.0f || q[k].hv >= 1.0f;
         }
@@ -299,7 +300,8 @@ __device__ __forceinline__ void finish(const FrameDesc& fd, const taa_uniforms_t
         f3 hc = rgb_to_ycocg(acc);
         // rejection (taa.comp:787-823)
         bool rejected = p.outside || p.masked;
-        if (lin_thr > 0.0f ? linear_depth_reject(p.pd, p.expected, near, far, lin_thr) : fabsf(p.pd - p.expected) > 0.1f * (1.0f - p.pd)) rejected = true;
+        if (G::PLAIN) {
+        } else if (lin_thr > 0.0f ? linear_depth_reject(p.pd, p.expected, near, far, lin_thr) : fabsf(p.pd - p.expected) > 0.1f * (1.0f - p.pd)) rejected = true;
         // clipAabb (taa.comp:323-345) towards the box's centre c, half size e
         f3 cur;
         bool found;
@@ -328,7 +330,7 @@ __device__ __forceinline__ void finish(const FrameDesc& fd, const taa_uniforms_t
         const float ld = fmaxf(fmaxf(lc, lh), 0.2f);
         const float diff = FA ? fabsf(lc - lh) * rcp_fast(ld) : fabsf(lc - lh) / ld;
         const float wl = 1.0f - diff;
-        float ab = gmix(a_max, a_min, wl * wl);
+        float ab = G::PLAIN ? P.mAlpha : gmix(a_max, a_min, wl * wl);
         if (!found) ab = ab * 0.0f;  // alpha * beta: beta is 0 where no sample was found, unless rejected or reset
         if (rejected) ab = a_reject;
         if (reset) ab = 1.0f;

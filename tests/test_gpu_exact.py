@@ -79,6 +79,31 @@ def test_default_block_equals_the_general_form(W, H, odd):
         both_forms(w, U, W, H, W + pad, (color, depth, vel4, hist, prev), FMT_RGBA16F, cas_for(w, W, H) if cas else None)
 
 
+def plain_params():
+    p = workload("c2")["params"]()
+    p.mVelocitySampleMode = p.mDepthCulling = p.mLumaWeightingLottes = p.mRejectOutside = 0
+    return p
+
+
+# without CAS one row a thread below 800 regions (the first three sizes), two rows above and with CAS
+@pytest.mark.parametrize("W,H,motion,odd", [(1, 1, 0, False), (33, 17, 6, True), (95, 61, 40, False), (1281, 721, 6, True), (31, 24001, 4, False)])
+@pytest.mark.parametrize("fmt", [FMT_RGBA16F, FMT_RGBA32F])
+def test_plain_form_equals_the_general_form(W, H, motion, odd, fmt):
+    for k, (cas, pad, reset, split) in enumerate([(True, 0, 0, 0), (False, 3, 0, 0), (True, 5, 0, W // 3), (False, 0, 1, 0)]):
+        print(f"case plain {W}x{H} fmt {fmt} cas {cas} pad {pad} reset {reset} split {split}", flush=True)
+        w = workload("c2", fmt=fmt, vel=VEL_RG16F if fmt == FMT_RGBA16F else VEL_RG32F)
+        U = uniforms_for(w, 1, (0.3 / W, -0.4 / H), params=plain_params())
+        U.mResetHistory, U.splitScreen, U.splitX = reset, int(split > 0), split
+        both_forms(w, U, W, H, W + pad, inputs(W, H, W, H, W + pad, W + pad, fmt, motion, odd, 171 + k), fmt, cas_for(w, W, H) if cas else None)
+
+
+@pytest.mark.parametrize("fmt", [FMT_RGBA16F, FMT_RGBA32F])
+def test_plain_batches(fmt, monkeypatch):
+    import test_gpu_upscale as t
+    monkeypatch.setattr(t, "uniforms_for", lambda w, f, j: uniforms_for(w, f, j, params=plain_params()))
+    batches([((480, 270), (480, 270)), ((33, 65), (33, 65))], fmt, ARITH_FP32)
+
+
 @pytest.mark.parametrize("specs", [[((480, 270), (480, 270)), ((640, 361), (640, 361)), ((33, 65), (33, 65))],
                                    [((160, 90), (160, 90)), ((95, 61), (95, 61))]])
 @pytest.mark.parametrize("fmt", [FMT_RGBA16F, FMT_RGBA32F])
@@ -123,3 +148,37 @@ def test_mask_equals_the_general_form(W, H, odd, fmt, arith):
         normals = (cells[..., None].float() + 0.2 * torch.rand(H, spl, 4, generator=g, device="cuda")).contiguous()
         old = torch.where(torch.rand(H, pitch, generator=g, device="cuda") < 0.1, (3 << 16) | 2, 0).to(torch.int32)
         both_forms(w, U, W, H, pitch, images, fmt, cas_for(w, W, H) if cas else None, arith, (material, prev.contiguous(), normals, old))
+
+
+@pytest.mark.parametrize("lo,W,H", [((960, 541), 960, 541), ((480, 270), 961, 541)])
+@pytest.mark.parametrize("fmt,arith", [(FMT_RGBA16F, ARITH_FP16), (FMT_RGBA16F, ARITH_FP32), (FMT_RGBA32F, ARITH_FP32)])
+def test_images_at_any_element(lo, W, H, fmt, arith):
+    """Images that begin one element into their allocation give the results of aligned ones."""
+    print(f"case alignment {lo} -> {W}x{H} fmt {fmt} arith {arith}", flush=True)
+    w = workload("c2", fmt=fmt, vel=VEL_RG16F if fmt == FMT_RGBA16F else VEL_RG32F)
+    U = uniforms_for(w, 1, (0.2 / W, 0.1 / H))
+    U.mUpsampling = int(lo != (W, H))
+    K = cas_for(w, W, H)
+    images = inputs(*lo, W, H, lo[0], W, fmt, 4, False, 7)
+
+    def moved(t, by):
+        s = torch.zeros(t.numel() + by, dtype=t.dtype, device="cuda")
+        s[by:] = t.reshape(-1)
+        return s
+
+    out = []
+    for by in (0, 1):
+        color, depth, vel, hist, prev = ts = [moved(t, by) for t in images]
+        screen, new = torch.zeros_like(hist), torch.zeros_like(hist)
+        at = lambda t: t.data_ptr() + by * t.element_size()
+        img = FrameImages()
+        img.color, img.depth, img.velocity, img.history, img.history_depth = [at(t) for t in ts]
+        img.result_history, img.result_screen = at(new), at(screen)
+        img.width, img.height, img.pitch = W, H, W
+        img.input_width, img.input_height, img.input_pitch = lo[0], lo[1], lo[0]
+        img.color_format, img.velocity_format = fmt, w["vel"]
+        check(lib().taa_resolve_frame(C.byref(U), C.byref(img), C.byref(K), arith, None))
+        torch.cuda.synchronize()
+        out.append((screen[by:], new[by:]))
+    assert_same_bits(out[0][0], out[1][0], "screen")
+    assert_same_bits(out[0][1], out[1][1], "history")
