@@ -208,11 +208,42 @@ int kernel_for(const taastar::FrameDesc& fd, const taa_uniforms_t& U, int param_
     return TAA_KERNEL_EXACT;
 }
 
+// Launch the one-size resolve of a frame whose columns and parameter block are set: the kernel of its arithmetic, storage and
+// parameters, on the tiles of its class's table entry (`shape`, -1: none). Returns a hipError_t as int.
+int launch_one_size(taastar::FrameDesc fd, const taa_uniforms_t& U, int arith, int shape, void* stream) {
+    const bool cas = fd.cas_on != 0, s16 = fd.color_fmt == TAA_FMT_RGBA16F;
+    const int def = shape >= 0 ? shape : default_shape(fd.W, fd.H, cas);
+    const taastar::TileShapeDef s = shape_def(def, cas);
+    fd.tiles_x = taastar::tiles_for(fd.x_end - fd.x_begin, s.tw);
+    fd.tiles_y = taastar::tiles_for(fd.H, s.th);
+    const bool fast = arith == TAA_ARITH_FP16 && taastar::fast_path_supported(fd, U, fd.param_idx);
+    const bool exact_default = arith == TAA_ARITH_FP32 && taastar::default_exact_form(fd, U, fd.param_idx);
+    if ((fast && s16) || exact_default) {
+        const int form = exact_default ? taastar::kDefaultExact : taastar::window_form(fd, U, fd.param_idx);
+        taastar::tile_window(fd, 2);
+        const long long n16 = (long long)fd.tiles_x * fd.tiles_y;
+        taastar::tile_window(fd, 4);
+        const long long n32 = (long long)fd.tiles_x * fd.tiles_y;
+        taastar::tile_window(fd, shape >= 0 ? taastar::kWindowRows[shape] : taastar::window_rows(n16, n32, cas, form));
+        if (exact_default && fd.rows == 4) taastar::tile_window(fd, 2);
+        return taastar::launch_window(fd, U, form, stream);
+    }
+    if (fast) return taastar::launch_resolve_fast(fd, U, def, stream);
+    taastar::FrameDesc p = fd;
+    taastar::tile_production(p, taastar::kProd256x2);
+    const long long n16 = (long long)p.tiles_x * p.tiles_y;
+    if (taastar::exact_prod_form(fd, U) && n16 >= taastar::exact_workgroups(cas, s16)) return taastar::launch_exact(p, U, false, stream);
+    if (taastar::exact_plain_form(fd, U)) {
+        taastar::tile_production(p, taastar::plain_variant(n16, cas));
+        return taastar::launch_exact(p, U, true, stream);
+    }
+    return taastar::launch_resolve(fd, U, def, arith, stream);
+}
+
 // Launch the resolve over [x_begin, x_end) with the given parameter block.
 int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, int x_end, int param_idx, int arith, void* stream,
                  const taastar::SegDesc* sg = nullptr) {
     if (x_end <= x_begin) return TAA_OK;
-    const bool cas = fd.cas_on != 0;
     if (sg) {  // segmentation mask: its own kernels, tiled by the launcher
         fd.x_begin = x_begin;
         fd.x_end = x_end;
@@ -223,48 +254,16 @@ int launch_range(taastar::FrameDesc fd, const taa_uniforms_t& U, int x_begin, in
         if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
         return TAA_OK;
     }
-    const int shape = selected_shape(fd.W, fd.H, fd.color_fmt, arith, cas);
-    const taastar::TileShapeDef s = shape_def(shape, cas);
     fd.x_begin = x_begin;
     fd.x_end = x_end;
     fd.param_idx = param_idx;
-    fd.tiles_x = taastar::tiles_for(x_end - x_begin, s.tw);
-    fd.tiles_y = taastar::tiles_for(fd.H, s.th);
     if (fd.up || U.mUpsampling) {  // upsampling path: the launcher tiles by its form's own shape
         fd.up = 1;
         const int e = taastar::upscale_form(fd, U) ? taastar::launch_upscale(fd, U, arith, stream) : taastar::launch_resolve_up(fd, U, arith, stream);
         if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
         return TAA_OK;
     }
-    int e;
-    const bool fast = arith == TAA_ARITH_FP16 && taastar::fast_path_supported(fd, U, param_idx);
-    const bool exact_default = arith == TAA_ARITH_FP32 && taastar::default_exact_form(fd, U, param_idx);
-    if (fast || exact_default) {
-        if (fd.color_fmt == TAA_FMT_RGBA16F) {
-            const int form = exact_default ? taastar::kDefaultExact : taastar::window_form(fd, U, param_idx);
-            const int tuned = tuned_shape(fd.W, fd.H, fd.color_fmt, arith, cas);
-            taastar::tile_window(fd, 2);
-            const long long n16 = (long long)fd.tiles_x * fd.tiles_y;
-            taastar::tile_window(fd, 4);
-            const long long n32 = (long long)fd.tiles_x * fd.tiles_y;
-            taastar::tile_window(fd, tuned >= 0 ? taastar::kWindowRows[tuned] : taastar::window_rows(n16, n32, cas, form));
-            if (exact_default && fd.rows == 4) taastar::tile_window(fd, 2);
-            e = taastar::launch_window(fd, U, form, stream);
-        } else {
-            e = taastar::launch_resolve_fast(fd, U, shape, stream);
-        }
-    } else {
-        taastar::FrameDesc p = fd;
-        taastar::tile_production(p, taastar::kProd256x2);
-        const long long n16 = (long long)p.tiles_x * p.tiles_y;
-        if (taastar::exact_prod_form(fd, U) && n16 >= taastar::exact_workgroups(cas, fd.color_fmt == TAA_FMT_RGBA16F)) {
-            e = taastar::launch_exact(p, U, false, stream);
-        } else if (taastar::exact_plain_form(fd, U)) {
-            taastar::tile_production(p, taastar::plain_variant(n16, cas));
-            e = taastar::launch_exact(p, U, true, stream);
-        } else
-            e = taastar::launch_resolve(fd, U, shape, arith, stream);
-    }
+    const int e = launch_one_size(fd, U, arith, tuned_shape(fd.W, fd.H, fd.color_fmt, arith, fd.cas_on != 0), stream);
     if (e != 0) return hip_fail((hipError_t)e, "resolve launch");
     return TAA_OK;
 }
@@ -1301,14 +1300,7 @@ int32_t taa_autotune(taa_ctx_t* c, int32_t w, int32_t h, int32_t fmt, int32_t ar
     int best = -1;
     float best_t = 1e30f;
     for (int s = 0; s < taastar::kNumShapes; ++s) {
-        const taastar::TileShapeDef sd = shape_def(s, cas != 0);
-        fd.tiles_x = taastar::tiles_for(w, sd.tw);
-        fd.tiles_y = taastar::tiles_for(h, sd.th);
-        const bool fast = arith == TAA_ARITH_FP16 && taastar::fast_path_supported(fd, U, 0);
-        auto go = [&]() {
-            if (fast) taastar::launch_resolve_fast(fd, U, s, st);
-            else taastar::launch_resolve(fd, U, s, arith, st);
-        };
+        auto go = [&]() { launch_one_size(fd, U, arith, s, st); };
         for (int i = 0; i < 3; ++i) go();
         hipEventRecord(e0, st);
         for (int i = 0; i < iters; ++i) go();

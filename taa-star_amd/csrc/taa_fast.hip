@@ -571,6 +571,7 @@ hipError_t launch_fast_g(const FrameDesc& fd, const taa_uniforms_t& U, int shape
 }
 
 int launch_resolve_fast(const FrameDesc& fd, const taa_uniforms_t& U, int shape, void* stream) {
+    if (fd.color_fmt != TAA_FMT_RGBA32F) return (int)hipErrorInvalidValue;  // RGBA16F: launch_window
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool insp = fd.inspect != nullptr;
     hipError_t e;
