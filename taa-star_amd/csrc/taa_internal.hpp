@@ -136,18 +136,20 @@ int launch_batch_fast(const BatchEntry* d_entries, int n_entries, int total_tile
 
 // The FP16-storage form of that kernel (taa_window.hip): a workgroup resolves a region of 32 columns x
 // 32 rows (fd.rows 4: 256 threads, four rows of a column each) or 16 rows (2: 256 threads, two rows
-// each; 1: 512 threads, one row each), of which fused CAS keeps the inner part.
+// each; 1: 512 threads, one row each, and without CAS, where there is no ring, 256 threads and 8 rows, whose smaller
+// workgroups spread evenly: 720x405 6.5 us against 9.0), of which fused CAS keeps the inner part.
 inline void tile_window(FrameDesc& fd, int rows) {
     const int ring = fd.cas_on ? 2 : 0;
     fd.rows = rows;
     fd.tiles_x = tiles_for(fd.x_end - fd.x_begin, 32 - ring);
-    fd.tiles_y = tiles_for(fd.H, (rows == 4 ? 32 : 16) - ring);
+    fd.tiles_y = tiles_for(fd.H, (rows == 4 ? 32 : rows == 1 && !ring ? 8 : 16) - ring);
 }
 // rows a thread of a class whose tile shape was tuned or selected (kShapesCas / kShapesPlain index)
 constexpr int kWindowRows[kNumShapes] = {1, 2, 4, 2};
 // Rows a thread for a launch of n16 workgroups on 16-row regions, n32 on 32-row ones (us a frame, FP16 storage
 // and arithmetic, three states in turn, rows 1 / 2 / 4). A launch that leaves the device part empty takes the most
-// threads: CAS 640x360 7.2 / 7.9 / 9.8, without CAS 800x450 7.3 / 8.0 / 10.2, but CAS 800x450 (891 workgroups)
+// threads: CAS 640x360 7.7 / 7.9 / 9.8, without CAS 800x450 7.3 / 8.0 / 10.2; in the range 480x270 to 720x405 with CAS
+// the tile kernel before this one took 0.3 to 0.7 less, but CAS 800x450 (891 workgroups)
 // 9.9 / 9.6 / 11.1. With CAS the 32-row region resolves 14% ring texels instead of 22% and wins once its workgroups
 // fill the device (five on each of 256 CUs): 1280x720 16.9 / 16.7 / 19.6, 1600x900 23.9 / 23.0 / 22.8, 3840x2160
 // 119 / 115 / 106. Without CAS there is no ring (2560x1440 55.1 / 45.6 / 47.8), and the reference's default block
@@ -207,7 +209,8 @@ inline int up_box_offset(int w, int h, int rows, bool s16) {
     const int most = staged > window ? staged : window;
     return ((most > resolved ? most : resolved) + 15) & ~15;
 }
-// Whether it takes this frame: with 1.4 (FP16 storage) or 1.6 (FP32 storage) output texels an input texel, where sharing
+// Whether it takes this frame: with 1.4 (FP16 storage) or 1.6 (FP32 storage; 1.8 below 2500 workgroups, and without CAS
+// from 600 on: 480x270 at 1.5 times the input 7.0 and 7.9 us) output texels an input texel, where sharing
 // an input texel's box among them pays for the larger LDS (us, the general kernel's production form and this one: FP16
 // 3840x2160 at 1.15 times the input's size 197 and 210, at 1.2 196 and 182; FP32 1920x1080 at 1.25 68 and 66, at 1.3 68 and
 // 60, 3840x2160 at 1.25 256 and 263).

@@ -307,8 +307,13 @@ void for_geometry(int variant, bool cas, bool s16, bool fa, F&& f) {
 }  // namespace
 
 bool upscale_form(const FrameDesc& fd, const taa_uniforms_t& U) {
+    if (fd.Wl > fd.W || fd.Hl > fd.H || !prod_params(fd, U)) return false;
     const long long out = (long long)fd.W * fd.H, in = (long long)fd.Wl * fd.Hl;
-    return fd.Wl <= fd.W && fd.Hl <= fd.H && out * 10 >= in * (fd.color_fmt == TAA_FMT_RGBA16F ? 14 : 16) && prod_params(fd, U);
+    if (fd.color_fmt == TAA_FMT_RGBA16F) return out * 10 >= in * 14;
+    FrameDesc p = fd;
+    tile_production(p, kProd256x2);
+    const long long n16 = (long long)p.tiles_x * p.tiles_y;
+    return out * 10 >= in * (n16 < 2500 ? 18 : 16) && (fd.cas_on || n16 >= 600);
 }
 
 int upscale_lds(const FrameDesc& fd, int variant) {

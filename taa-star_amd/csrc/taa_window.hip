@@ -73,7 +73,8 @@ struct WinGeo {
         alignas(16) unsigned char win[kWin > kDv ? kWin : kDv];  // depth and velocity until the window replaces them
         alignas(16) float2 c01[NS];                              // Y, Co; in the end the resolved texels for the fused CAS
         alignas(8) float c2[NS];                                 // Cg
-        __device__ uint2* res() { return reinterpret_cast<uint2*>(c01); }
+        uint2 own[WIN || !CAS ? 1 : RW * RH];  // without the window LDS is no limit: a place of their own saves a barrier
+        __device__ uint2* res() { return WIN ? reinterpret_cast<uint2*>(c01) : own; }
         float ux[SW], uy[SH];
         alignas(16) int4 box[NT / 64];
     };
@@ -105,23 +106,30 @@ __device__ __forceinline__ void resolve_window(const FrameDesc& fd, const taa_un
     const int x0 = fd.x_begin + tx * G::TW - G::RA, y0 = ty * G::TH - G::RA;  // the region's first texel
     const int tid = (int)threadIdx.x, rx = tid & 31, rg = (tid >> 5) * RPT;
 
-    const int sample_mode = G::CLOSEST == kAny ? scalar_now(P.mVelocitySampleMode) : G::CLOSEST * 2;
-    const bool ycocg = opt(G::YCOCG, flag(P.mUseYCoCg));
+    // parameters read here, ahead of their phases; one row a thread (all workgroups start at once) has its first loads under way sooner
+    // without waiting for them
+    auto pin = [](auto v) {
+        if constexpr (G::RPT > 1) return scalar_now(v);
+        else return v;
+    };
+    auto pinned_flag = [&](int v) { return pin(v) != 0; };
+    const int sample_mode = G::CLOSEST == kAny ? pin(P.mVelocitySampleMode) : G::CLOSEST * 2;
+    const bool ycocg = opt(G::YCOCG, pinned_flag(P.mUseYCoCg));
     const bool closest_mode = sample_mode == 2;
-    const int rect = G::RECT == kAny ? scalar_now(P.mColorClampingOrClipping) : G::RECT;
-    const bool lottes = opt(G::LOTTES, flag(P.mLumaWeightingLottes));
-    const bool reject_out = opt(G::OUTSIDE, flag(P.mRejectOutside));
-    const bool depth_cull = opt(G::CULL, flag(P.mDepthCulling));
-    const bool reset = flag(U.mResetHistory);
-    const bool var_clip = opt(G::VAR, flag(P.mVarianceClipping));
-    const bool cr_hist = G::CR == kAny ? scalar_now(P.mInterpolationMode) == 2 : G::CR != 0;
-    const bool ghost = opt(G::OPTIONS, flag(P.mDynamicAntiGhosting));
-    const bool vel_alpha = opt(G::OPTIONS, flag(P.mVelBasedAlpha)), near_clamp = opt(G::OPTIONS, flag(P.mReduceBlendNearClamp));
+    const int rect = G::RECT == kAny ? pin(P.mColorClampingOrClipping) : G::RECT;
+    const bool lottes = opt(G::LOTTES, pinned_flag(P.mLumaWeightingLottes));
+    const bool reject_out = opt(G::OUTSIDE, pinned_flag(P.mRejectOutside));
+    const bool depth_cull = opt(G::CULL, pinned_flag(P.mDepthCulling));
+    const bool reset = pinned_flag(U.mResetHistory);
+    const bool var_clip = opt(G::VAR, pinned_flag(P.mVarianceClipping));
+    const bool cr_hist = G::CR == kAny ? pin(P.mInterpolationMode) == 2 : G::CR != 0;
+    const bool ghost = opt(G::OPTIONS, pinned_flag(P.mDynamicAntiGhosting));
+    const bool vel_alpha = opt(G::OPTIONS, pinned_flag(P.mVelBasedAlpha)), near_clamp = opt(G::OPTIONS, pinned_flag(P.mReduceBlendNearClamp));
     const bool longest = EXT && sample_mode == 1;
-    const int use_velocity = G::DEF ? 1 : EXT ? scalar_now(P.mUseVelocityVectors) : 2;
-    const float gamma = scalar_now(P.mVarClipGamma), a_plain = scalar_now(P.mAlpha), a_max = scalar_now(P.mMaxAlpha),
-                a_min = scalar_now(P.mMinAlpha), a_reject = scalar_now(P.mRejectionAlpha), peak = scalar_now(__uint_as_float(fd.cas_peak_bits));
-    const float near = scalar_now(U.mCamNearPlane), far = scalar_now(U.mCamFarPlane), lin_thr = scalar_now(U.pad1);
+    const int use_velocity = G::DEF ? 1 : EXT ? pin(P.mUseVelocityVectors) : 2;
+    const float gamma = pin(P.mVarClipGamma), a_plain = pin(P.mAlpha), a_max = pin(P.mMaxAlpha),
+                a_min = pin(P.mMinAlpha), a_reject = pin(P.mRejectionAlpha), peak = pin(__uint_as_float(fd.cas_peak_bits));
+    const float near = pin(U.mCamNearPlane), far = pin(U.mCamFarPlane), lin_thr = pin(U.pad1);
     const bool lin_depth = lin_thr > 0.0f;
     const float fW = (float)W, fH = (float)H;
     const Image color(fd.color, fd.pitch, W, H, 8), depths(fd.depth, fd.pitch, W, H, 4), velocity(fd.velocity, fd.pitch, W, H, (int)sizeof(VelT)),
@@ -691,7 +699,7 @@ __device__ __forceinline__ void resolve_window(const FrameDesc& fd, const taa_un
     // ---- 5. fused CAS: left and right neighbours from LDS, upper and lower ones of the thread's own column where it
     // has them; at the image's border the missing neighbour is the texel itself
     if constexpr (G::CAS) {
-        __syncthreads();  // every thread is done with the staged colours
+        if constexpr (G::WIN) __syncthreads();  // every thread is done with the staged colours
         uint2* const res = sm.res();
 #pragma unroll
         for (int k = 0; k < RPT; ++k) res[(rg + k) * 32 + rx] = hbs[k];
@@ -786,7 +794,7 @@ void launch_window_batch_f(const BatchEntry* e, int n, int total, int form, hipS
 template <bool CAS, bool INSP>
 void launch_window_r(const FastArgs& a, int form, hipStream_t st) {
     switch (a.fd.rows) {
-        case 1: launch_window_f<512, 1, CAS, INSP>(a, form, st); break;
+        case 1: launch_window_f<CAS ? 512 : 256, 1, CAS, INSP>(a, form, st); break;
         case 2: launch_window_f<256, 2, CAS, INSP>(a, form, st); break;
         default: launch_window_f<256, 4, CAS, INSP>(a, form, st); break;
     }
@@ -795,7 +803,7 @@ void launch_window_r(const FastArgs& a, int form, hipStream_t st) {
 template <bool CAS>
 void launch_window_batch_r(const BatchEntry* e, int n, int total, int rows, int form, hipStream_t st) {
     switch (rows) {
-        case 1: launch_window_batch_f<512, 1, CAS>(e, n, total, form, st); break;
+        case 1: launch_window_batch_f<CAS ? 512 : 256, 1, CAS>(e, n, total, form, st); break;
         case 2: launch_window_batch_f<256, 2, CAS>(e, n, total, form, st); break;
         default: launch_window_batch_f<256, 4, CAS>(e, n, total, form, st); break;
     }
