@@ -71,9 +71,9 @@ enum { TAA_VEL_RG32F = 0, TAA_VEL_RG16F = 1, TAA_VEL_RGBA32F = 2, TAA_VEL_RGBA16
 enum { TAA_ARITH_FP32 = 0, TAA_ARITH_FP16 = 1 };
 /* the kernel a resolve runs (taa_resolve_kernel) */
 enum {
-    TAA_KERNEL_EXACT = 0,    /* FP32 arithmetic in taa.comp's operation order (k_resolve)      */
-    TAA_KERNEL_FP16 = 1,     /* the FP16-arithmetic throughput kernel (k_resolve_fast)         */
-    TAA_KERNEL_UPSAMPLE = 2, /* the exact FP32 upsampling resolve (k_resolve_up)               */
+    TAA_KERNEL_EXACT = 0,    /* FP32 arithmetic in taa.comp's operation order                  */
+    TAA_KERNEL_FP16 = 1,     /* the FP16-arithmetic throughput kernel                          */
+    TAA_KERNEL_UPSAMPLE = 2, /* the exact FP32 upsampling resolve                              */
     TAA_KERNEL_UPSAMPLE_FP16 = 3 /* the upsampling resolve with the FP16 path's arithmetic      */
 };
 
@@ -457,7 +457,8 @@ int32_t taa_batch_submit(taa_ctx_t* ctx, int32_t n, const taa_batch_item_t* item
  * class's shape, several take the shape tuned for the largest class of at most their total
  * pixel count (a launch over many frames behaves like one frame of their total size), or the
  * default shape when it resolves 2% fewer texels over the batch's frames. Frames on the FP16 kernel with
- * RGBA16F storage are tiled by the launch's size alone. */
+ * RGBA16F storage, on the fixed forms of the exact kernel and on the upsampling kernel are tiled by the launch's
+ * size alone. */
 typedef struct taa_batch_plan taa_batch_plan_t;
 int32_t taa_batch_plan_create(taa_ctx_t* ctx, int32_t n, const taa_batch_item_t* items,
                               int32_t arith, taa_batch_plan_t** out);
@@ -488,7 +489,9 @@ int32_t taa_autotune(taa_ctx_t* ctx, int32_t width, int32_t height, int32_t colo
  * or for frames of fewer 30x30 tiles than the device holds workgroups at once, 30x14 and below
  * 512 such tiles 14x14).
  * The FP16 kernel with RGBA16F storage resolves 32-column regions instead: entries 0 to 3 select one,
- * two, four and two rows a thread. */
+ * two, four and two rows a thread. The exact arithmetic's production and plain parameter sets run on 32-column
+ * regions of their own, whatever the entry, where that is the faster kernel; its default block on RGBA16F takes
+ * entry 0 as one row a thread and the others as two. */
 int32_t taa_tile_shape_select(int32_t width, int32_t height, int32_t color_format, int32_t arith,
                               taa_bool32 cas, int32_t index);
 /* The shape index the table holds for a frame class. */
