@@ -12,7 +12,8 @@
 // eight of them a wave, against 4.5-5 clocks for an LDS read. So a workgroup first finds the positions of all its
 // texels (1, 2), then loads the rectangle their footprints cover into LDS once, two texels a lane (3), and
 // filters from there (4): the L1's busy time at 4K falls from 168,000 to 106,000 clocks. A tile whose
-// footprints lie too far apart for the window (48 columns, the region's height + 16 rows) reads texel by texel.
+// footprints lie too far apart for the window (48 columns, the region's height + 16 rows) reads them from memory; a scene in which
+// neighbouring objects move 24 texels apart everywhere runs 149 us a 4K frame so, 12 more than the tile kernel that held footprints in registers.
 // A thread owns consecutive rows of one column, so the 3x3 sums and the closest-depth search share its rows
 // (a row's three texels are summed and compared once, not three times), the CAS takes its upper and
 // lower neighbours from registers, and row offsets are scalar: 1,440 VALU instructions a wave of 4 x 64 texels against
@@ -518,7 +519,18 @@ __device__ __forceinline__ void resolve_window(const FrameDesc& fd, const taa_un
                     const uint2 e[4] = {w[j * G::WP], w[j * G::WP + 1], w[j * G::WP + 2], w[j * G::WP + 3]};
                     add_row(e, wy.w[j]);
                 }
-            } else {  // the tile's footprints lie too far apart for the window: texel by texel from memory
+            } else if (__builtin_amdgcn_ballot_w64(q[k].kx < 1 || q[k].kx > W - 3 || q[k].ky < 1 || q[k].ky > H - 3) == 0) {
+                // the tile's footprints lie too far apart for the window (motion that differs by more than its margin): from
+                // memory, a row's two 16-byte loads at a time (two rows at a time cost registers everywhere: 3840x2160 113 us, not 108)
+                uint32_t o = ((uint32_t)(q[k].ky - 1) * pitch + (uint32_t)(q[k].kx - 1)) * 8u;
+#pragma unroll 1
+                for (int j = 0; j < 4; ++j) {
+                    const u32x4 a = history.ld4(o, 0u), b = history.ld4(o + 16u, 0u);
+                    const uint2 e[4] = {make_uint2(a.x, a.y), make_uint2(a.z, a.w), make_uint2(b.x, b.y), make_uint2(b.z, b.w)};
+                    add_row(e, j == 0 ? wy.w[0] : j == 1 ? wy.w[1] : j == 2 ? wy.w[2] : wy.w[3]);
+                    o += pitch * 8u;
+                }
+            } else {  // ... and over the image's edge: texel by texel, clamped
 #pragma unroll 1
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t r = (uint32_t)clampi(q[k].ky - 1 + j, 0, H - 1) * pitch;
